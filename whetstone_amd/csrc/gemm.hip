@@ -1173,10 +1173,11 @@ GemmPlan plan_gemm(int in_f, int out_f, int n, bool hier = true, int rows = 0, b
   GemmPlan p;
   if (rows <= 0) rows = out_f;
   const int pn = plan_n > 0 && plan_n < n ? plan_n : n;
-  // (The wide tiles address x with 32-bit byte offsets.)
+  // (The wide tiles address x with 32-bit byte offsets, and step through it
+  // 64 columns at a time: in_f must be whole steps.)
   const int tm = gemm_tiles_mode();
   const int rows_t256 = ((rows + GW_BM - 1) / GW_BM) * ((pn + 255) / 256);
-  p.wide = hier && tm > 0 && in_f >= GW_KC &&
+  p.wide = hier && tm > 0 && in_f % GW_KC == 0 &&
            (tm == 2 || in_f >= 2048 || rows >= 4096 || rows_t256 >= wst_cu_count() / 2) &&
            (size_t)n * in_f * 2 < ((size_t)1 << 31);
   // Wide tiles of 128 tokens for the split-K shapes (256-token tiles fewer
