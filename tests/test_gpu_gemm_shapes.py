@@ -45,3 +45,84 @@ def test_gemm_odd_group_counts(orc, wk, in_f, out_f, n, accum):
     if accum:
         ref = ref + y0.reshape(n, out_f)
     _check(y.numpy().astype(np.float64).reshape(n, out_f), x, w, ref)
+
+
+# rows of whole 128-column steps: one step, an odd and an even count of them;
+# one row, a row tile's edge and one past it; one token, a token tile's edge
+# and one past it; K split (long rows) with and without the accumulate
+@pytest.mark.parametrize("in_f,out_f,n,accum", [(128, 1, 1, False), (256, 256, 128, True),
+                                                (384, 257, 129, False), (896, 127, 127, True),
+                                                (1152, 130, 70, False), (4864, 896, 256, True),
+                                                (3584, 1056, 1000, False), (9216, 33, 200, True)])
+def test_gemm_whole_step_rows(orc, wk, in_f, out_f, n, accum):
+    print(f"gemm {in_f} -> {out_f}, {n} tokens", flush=True)
+    lin, w, x, xd, bias, bd = _operands(orc, wk, in_f, out_f, n, 62)
+    y0 = orc.fixture_normal(62, 4, (n + 1) * out_f, 1.0)
+    y = wk.DeviceBuffer.from_array(y0.copy())
+    ffi.call("wst_gemm_int4_hier", lin.qw.ptr, lin.si.ptr, lin.sb.ptr, xd.ptr, bd.ptr, y.ptr, in_f,
+             out_f, n, int(accum))
+    got = y.numpy().astype(np.float64).reshape(n + 1, out_f)
+    ref = x @ w.T + bias
+    if accum:
+        ref = ref + y0.reshape(n + 1, out_f)[:n]
+    _check(got[:n], x, w, ref)
+    assert np.array_equal(got[n], y0.reshape(n + 1, out_f)[n])  # nothing past the last token
+
+
+@pytest.mark.parametrize("in_f,inter,n", [(128, 1, 1), (256, 128, 128), (896, 161, 129),
+                                          (384, 700, 300)])
+def test_gemm_swiglu_whole_step_rows(orc, wk, in_f, inter, n):
+    print(f"gate|up {in_f} -> {inter}, {n} tokens", flush=True)
+    lin, w, x, xd, _, _ = _operands(orc, wk, in_f, 2 * inter, n, 63)
+    act = wk.DeviceBuffer.from_array(np.full((n + 1) * inter, 7.0, np.float16))
+    ffi.call("wst_gemm_hier_swiglu_chunk", lin.qw.ptr, lin.si.ptr, lin.sb.ptr, xd.ptr, act.ptr,
+             in_f, inter, n)
+    got = act.numpy().astype(np.float64).reshape(n + 1, inter)
+    gu = x @ w.T
+    err = 2.0 * 2.0 ** -11 * (np.abs(x) @ np.abs(w).T) + 1e-5
+    g, u = gu[:, :inter], gu[:, inter:]
+    silu = g / (1 + np.exp(-g))
+    # silu' <= 1.1: the products' errors through silu(g) * u, and the f16 store
+    bound = 1.1 * err[:, :inter] * np.abs(u) + np.abs(silu) * err[:, inter:]
+    bound = 1.1 * bound + 2.0 ** -10 * np.abs(silu * u) + 1e-4
+    worst = float(np.max(np.abs(got[:n] - silu * u) / bound))
+    assert worst <= 1.0, worst
+    assert np.all(got[n] == 7.0)
+
+
+@pytest.mark.parametrize("in_f,n_q,n_kv,hd,pos0,n,qk", [(3584, 28, 4, 128, 5, 2049, False),
+                                                        (896, 14, 2, 64, 3, 4000, True)])
+def test_gemm_rope_epilogue_equals_gemm_then_rope_cache(orc, wk, in_f, n_q, n_kv, hd, pos0, n, qk):
+    """Enough tokens that the projection runs unsplit on the big tiles, whose
+    epilogue rotates and appends: against the GEMM then wst_rope_cache_chunk,
+    bit for bit, at both head sizes (the last token tile ragged, the cache
+    ending at the last token)."""
+    print(f"rope epilogue hd {hd}, {n} tokens", flush=True)
+    out_f, max_seq = (n_q + 2 * n_kv) * hd, pos0 + n
+    lin = wk.QuantLinearHier(*(wk.DeviceBuffer(k, t) for k, t in (
+        (out_f * in_f // 8, np.uint32), (out_f * in_f // 32, np.uint8), (out_f, np.uint32))),
+        in_f, out_f)
+    ffi.call("wst_fixture_pack_hier", lin.qw.ptr, lin.si.ptr, lin.sb.ptr, in_f, 0, out_f, 64, 1, 0.02)
+    x = dev_f16(wk, f16(orc, orc.fixture_normal(64, 2, n * in_f, 1.0)))
+    b = dev_f16(wk, f16(orc, orc.fixture_normal(64, 3, out_f, 0.3)))
+    norms = [dev_f16(wk, f16(orc, 1.0 + orc.fixture_normal(64, 4 + i, hd, 0.1))) if qk else None
+             for i in range(2)]
+    qn, kn = (v.ptr if v is not None else None for v in norms)
+    c, s = orc.rope_table(max_seq, hd, 1e6)
+    cd, sd = wk.DeviceBuffer.from_array(c), wk.DeviceBuffer.from_array(s)
+    out = []
+    for fused in (False, True):
+        qkv = wk.DeviceBuffer(n * out_f, np.float32)
+        k, v = (wk.DeviceBuffer(n_kv * max_seq * hd, np.float16) for _ in range(2))
+        if fused:
+            ffi.call("wst_gemm_hier_rope_chunk", lin.qw.ptr, lin.si.ptr, lin.sb.ptr, x.ptr, b.ptr,
+                     qkv.ptr, in_f, k.ptr, v.ptr, cd.ptr, sd.ptr, n_q, n_kv, hd, pos0, n, max_seq,
+                     qn, kn, 1e-6)
+        else:
+            ffi.call("wst_gemm_int4_hier", lin.qw.ptr, lin.si.ptr, lin.sb.ptr, x.ptr, b.ptr,
+                     qkv.ptr, in_f, out_f, n, 0)
+            ffi.call("wst_rope_cache_chunk", qkv.ptr, k.ptr, v.ptr, cd.ptr, sd.ptr, n_q, n_kv, hd,
+                     pos0, n, max_seq, qn, kn, 1e-6)
+        out.append([t.numpy() for t in (qkv, k, v)])
+    for a, e in zip(*out):
+        assert np.array_equal(a.view(np.uint8), e.view(np.uint8))

@@ -35,6 +35,7 @@
 // * The fp16 form (wst_gemm_fp16, the lossless reference path) runs the same
 //   kernel with the W tile copied instead of dequantised.
 #include "common.hpp"
+#include "gemm_tile.hpp"
 
 #include <mutex>
 
@@ -351,7 +352,6 @@ __global__ __launch_bounds__(GM_THREADS) void gemm_mfma_kernel(
 //   0..31 of a tile are gate rows a0..a0+31 and rows 32..63 the up rows
 //   inter+a0.., and the epilogue writes act = f16(silu(gate) * up).
 #define GW_BM 64
-#define GW_ROPE_HD 64                   // head_dim of the RoPE epilogue: one tile's rows
 #define GW_KG 2
 #define GW_KC (GW_KG * HGROUP)          // 64 columns per step
 #define GW_KS (GW_KC + 8)               // W tile row stride in halves
@@ -395,83 +395,11 @@ struct GwShape {
 
 typedef float gm_f16v __attribute__((ext_vector_type(16)));
 
-// The qkv GEMM's RoPE epilogue (ROPE tiles, head_dim 64 = one tile's rows):
-// what gemm_reduce_rope_kernel does after an unsplit GEMM, per token.
-struct GwRope {
-  uint16_t *k_cache, *v_cache;
-  const float *cos_tab, *sin_tab;
-  const uint16_t *q_norm_w, *k_norm_w;
-  int n_q, n_kv, pos0, max_seq;
-  float eps;
-};
-
-// RT tokens of one head of 64, stage by stage so that the tokens' dependent
-// chains (cross-lane swap, norm reduction, square root) overlap: lane j holds
-// column j of each (the value after the GEMM and bias); q is QK-normed,
-// rotated and stored to its row, k stored to its row as computed and rotated
-// into the cache, v stored to its row and the cache. The arithmetic is
-// gemm_reduce_rope_kernel's NARROW form (column j in lane j, the rotation
-// partner over a 32-lane swap, the norm's pair sums over the wave), so the
-// two give the same bits. ok[u]: token u exists (uniform in the wave).
-template <int RT>
-__device__ __forceinline__ void gw_rope_tokens(const float (&mine)[RT], const bool (&ok)[RT],
-                                               const int (&tok)[RT], int h, float *__restrict__ y,
-                                               int row_stride, const GwRope &re,
-                                               const float (&c)[RT], const float (&s)[RT],
-                                               float gq1, float gq2, int lane) {
-  const int hd = GW_ROPE_HD;
-  const bool hi = lane >= 32;
-  int pos[RT];
-#pragma unroll
-  for (int u = 0; u < RT; ++u) pos[u] = min(max(re.pos0 + tok[u], 0), re.max_seq - 1);
-  if (h >= re.n_q + re.n_kv) {  // v
-    const int kvh = h - re.n_q - re.n_kv;
-#pragma unroll
-    for (int u = 0; u < RT; ++u)
-      if (ok[u]) {
-        y[(size_t)tok[u] * row_stride + h * hd + lane] = mine[u];
-        re.v_cache[((size_t)kvh * re.max_seq + pos[u]) * hd + lane] = f2h(mine[u]);
-      }
-    return;
-  }
-  const bool is_q = h < re.n_q;
-  float x1[RT], x2[RT];
-#pragma unroll
-  for (int u = 0; u < RT; ++u) {
-    const float other = __shfl_xor(mine[u], 32);
-    x1[u] = hi ? other : mine[u];
-    x2[u] = hi ? mine[u] : other;
-  }
-  if (is_q ? re.q_norm_w : re.k_norm_w) {
-    float ss[RT];
-#pragma unroll
-    for (int u = 0; u < RT; ++u) ss[u] = wave_sum(!hi ? fmaf(x1[u], x1[u], x2[u] * x2[u]) : 0.0f);
-#pragma unroll
-    for (int u = 0; u < RT; ++u) {
-      const float sc = 1.0f / sqrtf(ss[u] / (float)hd + re.eps);
-      x1[u] = x1[u] * sc * gq1;
-      x2[u] = x2[u] * sc * gq2;
-    }
-  }
-#pragma unroll
-  for (int u = 0; u < RT; ++u) {
-    if (!ok[u]) continue;
-    const float lo = rope_lo(x1[u], x2[u], c[u], s[u]), hv = rope_hi(x1[u], x2[u], c[u], s[u]);
-    float *row = y + (size_t)tok[u] * row_stride;
-    if (is_q) {
-      row[h * hd + lane] = hi ? hv : lo;
-    } else {
-      row[h * hd + lane] = mine[u];  // k as computed
-      re.k_cache[((size_t)(h - re.n_q) * re.max_seq + pos[u]) * hd + lane] = f2h(hi ? hv : lo);
-    }
-  }
-}
-
-template <bool HIER, bool SWI, int NWV, bool ROPE = false>
+template <bool HIER, bool SWI, int NWV>
 __global__ __launch_bounds__(64 * NWV, 1) void gemm_wide_kernel(
     const void *__restrict__ w, const uint8_t *__restrict__ si, const uint32_t *__restrict__ sb,
     const uint16_t *__restrict__ x, const uint16_t *__restrict__ bias, float *__restrict__ y,
-    float *__restrict__ ws, int in_f, int out_f, int n, int accum, int gps, GwRope re) {
+    float *__restrict__ ws, int in_f, int out_f, int n, int accum, int gps) {
 #pragma clang fp contract(off)
   static_assert(HIER, "the wide tiles take int4-hier weights");
   using S = GwShape<NWV>;
@@ -692,20 +620,6 @@ __global__ __launch_bounds__(64 * NWV, 1) void gemm_wide_kernel(
                  :: "memory");
   __syncthreads();
 
-  // RoPE epilogue: the rotation angles of the wave's tokens (every NWV-th of
-  // the tile's), loaded while the accumulators go through LDS.
-  constexpr int RTOK = ROPE ? BN / NWV : 1;
-  float rc[RTOK], rsn[RTOK];
-  if constexpr (ROPE) {
-    const int half = GW_ROPE_HD / 2, jj = lane & 31;
-#pragma unroll
-    for (int i = 0; i < RTOK; ++i) {
-      const int pos = min(max(re.pos0 + t0 + wave + i * NWV, 0), re.max_seq - 1);
-      rc[i] = re.cos_tab[(size_t)pos * half + jj];
-      rsn[i] = re.sin_tab[(size_t)pos * half + jj];
-    }
-  }
-
   // Epilogue through LDS, token-major: accumulator r of row tile a holds row
   // 32 a + 8 (r / 4) + 4 (lane / 32) + r % 4, token lane % 32 of the wave.
   float *ct = (float *)gw_lds;  // [BN][GW_CS]
@@ -717,34 +631,6 @@ __global__ __launch_bounds__(64 * NWV, 1) void gemm_wide_kernel(
       ct[(wave * 32 + l32) * GW_CS + row] = acc[a][r];
     }
   __syncthreads();
-  if constexpr (ROPE) {
-    // the tile's 64 rows are head h; each wave takes every NWV-th token
-    static_assert(!SWI && GW_BM == GW_ROPE_HD, "the RoPE tiles are one head of the plain GEMM");
-    const int h = r0 / GW_BM, half = GW_ROPE_HD / 2, jj = lane & 31;
-    const float bj = bias ? h2f(bias[r0 + lane]) : 0.0f;
-    const uint16_t *g = h < re.n_q ? re.q_norm_w : re.k_norm_w;
-    const float gq1 = g ? h2f(g[jj]) : 0.0f, gq2 = g ? h2f(g[jj + half]) : 0.0f;
-    constexpr int RT = 4;
-    static_assert(RTOK % RT == 0, "tokens in groups of four");
-#pragma unroll
-    for (int i0 = 0; i0 < RTOK; i0 += RT) {
-      float mine[RT], c[RT], sn[RT];
-      bool ok[RT];
-      int tok[RT];
-#pragma unroll
-      for (int u = 0; u < RT; ++u) {
-        const int tl = wave + (i0 + u) * NWV;
-        tok[u] = t0 + tl;
-        ok[u] = tok[u] < n;
-        mine[u] = ct[tl * GW_CS + lane];
-        if (bias) mine[u] += bj;
-        c[u] = rc[i0 + u];
-        sn[u] = rsn[i0 + u];
-      }
-      gw_rope_tokens<RT>(mine, ok, tok, h, y, out_f, re, c, sn, gq1, gq2, lane);
-    }
-    return;
-  }
   if constexpr (SWI) {
     uint16_t *act = (uint16_t *)y;
     const int a0 = r0 / 2;
@@ -1125,7 +1011,14 @@ void set_lds_attr() {
   }
 }
 
+// Register-dequantising tiles (gemm_tile.hpp): 256 rows x 128 tokens in four
+// waves of 64 x 128, and 128 rows x 128 tokens in eight waves of 32 x 64.
+using GtBig = GtShape<4, 1, 2, 4>;
+using GtSmall = GtShape<4, 2, 1, 2>;
+enum GemmTile { TILE_OLD = 0, TILE_BIG = 1, TILE_SMALL = 2 };
+
 struct GemmPlan {
+  int tile;  // GemmTile; TILE_OLD: the LDS tiles (wide or not, below)
   bool wide;
   int nwv;  // wide tiles: waves of 32 tokens (8: 256-token tiles, 4: 128)
   int bm, bn, kg;
@@ -1153,6 +1046,52 @@ static int gemm_bn_override() {
   return v;
 }
 
+// The register-dequantising tiles take int4-hier rows of whole 128-column
+// steps with 4-byte aligned index bytes, within their 32-bit offsets.
+bool tile_ok(const void *si, int in_f, int out_f, int rows, int n) {
+  const size_t lim = (size_t)1 << 31;
+  return gemm_tiles_mode() == 1 && in_f % GT_KC == 0 && !((uintptr_t)si & 3u) &&
+         (size_t)n * in_f * 2 < lim && (size_t)rows * (in_f / 2) < lim &&
+         (size_t)n * out_f * 4 < lim && out_f <= (1 << 20);
+}
+
+// Tile and K split by the time the most loaded CU takes: blocks per CU x steps
+// per block x the tile's step time, plus the tile's fixed part (launch,
+// first loads, stores) and the partials' traffic. Step and fixed times
+// measured over 896..18944-column rows and 256..4096 tokens: big 1.8 us and
+// 12 us, small 1.45 us and 7 us (two blocks on a CU take twice as long as one:
+// they share the matrix cores and the VALU), partials 4 TB/s. A split's
+// partials stay below max_part bytes.
+void plan_tile(GemmPlan &p, int in_f, int out_f, int rows, int pn, int n, bool may_split,
+               bool small_ok, size_t max_part) {
+  const int steps = in_f / GT_KC, cus = wst_cu_count();
+  float best = 0.0f;
+  p.tile = TILE_OLD;
+  for (int t = TILE_BIG; t <= (small_ok ? TILE_SMALL : TILE_BIG); ++t) {
+    const int bm = t == TILE_BIG ? GtBig::BM : GtSmall::BM;
+    const int bn = t == TILE_BIG ? GtBig::BN : GtSmall::BN;
+    const float step_us = t == TILE_BIG ? 1.8f : 1.45f, fixed_us = t == TILE_BIG ? 12.0f : 7.0f;
+    const int tiles = ((rows + bm - 1) / bm) * ((pn + bn - 1) / bn);
+    for (int want = 1; want <= (may_split ? GM_MAXSPLIT : 1) && want <= steps; ++want) {
+      const int sps = (steps + want - 1) / want, splits = (steps + sps - 1) / sps;
+      const size_t part = (size_t)splits * n * out_f * 4;
+      if (splits > 1 && part > max_part) break;
+      if (gemm_split_cap() > 0 && splits > gemm_split_cap()) break;
+      const float us = (float)((tiles * splits + cus - 1) / cus) * (float)sps * step_us + fixed_us +
+                       (splits > 1 ? 3.0f + (float)splits * (float)pn * (float)out_f * 8.0f / 4.0e6f
+                                   : 0.0f);
+      if (p.tile == TILE_OLD || us < best) {
+        best = us;
+        p.tile = t;
+        p.bm = bm;
+        p.bn = bn;
+        p.splits = splits;
+        p.gps = sps;  // steps of GT_KC columns
+      }
+    }
+  }
+}
+
 // Splits so that the grid covers the chip, each at least one step long.
 // rows: the weight matrix's row count (2 * inter for the SwiGLU form), which
 // with in_f and the plan's token count picks the tiles: the wide tiles for
@@ -1169,10 +1108,20 @@ static int gemm_bn_override() {
 // plan_n tokens gives it (the tiles are 64, 128 or 256 tokens, which divide
 // a chunk). 0: n itself.
 GemmPlan plan_gemm(int in_f, int out_f, int n, bool hier = true, int rows = 0, bool swi = false,
-                   int plan_n = 0) {
+                   int plan_n = 0, const void *si = nullptr,
+                   size_t max_part = (size_t)256 << 20) {
   GemmPlan p;
   if (rows <= 0) rows = out_f;
   const int pn = plan_n > 0 && plan_n < n ? plan_n : n;
+  if (hier && tile_ok(si, in_f, out_f, rows, n)) {
+    plan_tile(p, in_f, out_f, rows, pn, n, !swi, !swi, max_part);
+    p.wide = false;
+    p.nwv = 0;
+    p.kg = 0;
+    p.grid = dim3((unsigned)(((rows + p.bm - 1) / p.bm) * ((n + p.bn - 1) / p.bn)), p.splits, 1);
+    return p;
+  }
+  p.tile = TILE_OLD;
   // (The wide tiles address x with 32-bit byte offsets, and step through it
   // 64 columns at a time: in_f must be whole steps.)
   const int tm = gemm_tiles_mode();
@@ -1217,20 +1166,55 @@ GemmPlan plan_gemm(int in_f, int out_f, int n, bool hier = true, int rows = 0, b
   return p;
 }
 
+template <class S, int EPI>
+void launch_tile(const GemmPlan &p, const void *w, const void *si, const void *sb, const void *x,
+                 const void *bias, void *y, float *ws, int in_f, int out_f, int rows, int n,
+                 int accum, const GtRope &re) {
+  static bool attr = false;
+  if (!attr) {
+    (void)hipFuncSetAttribute((const void *)gemm_tile_kernel<S, EPI>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS);
+    attr = true;
+  }
+  // An XCD's blocks take consecutive tiles: row tiles vary fastest (few token
+  // tiles an XCD, every row) where x outweighs the packed weights, so that
+  // each XCD's L2 reads the larger operand once (0.5B o over 4096 tokens 16.3
+  // -> 14.9 us, qkv 24.2 -> 22.6 us).
+  const int rfast = (size_t)n * 2 * 16 > (size_t)rows * 9;
+  gemm_tile_kernel<S, EPI><<<p.grid, S::THREADS, S::LDS, WST_STREAM>>>(
+      w, (const uint8_t *)si, (const uint32_t *)sb, (const uint16_t *)x, (const uint16_t *)bias,
+      (float *)y, ws, in_f, out_f, n, accum, (n + S::BN - 1) / S::BN, (int)p.grid.x, p.gps, rfast,
+      re);
+}
+
 template <bool HIER, bool SWI>
 void launch_gemm(const GemmPlan &p, const void *w, const void *si, const void *sb, const void *x,
                  const void *bias, void *y, float *ws, int in_f, int out_f, int n, int accum) {
+  if constexpr (HIER) {
+    if (p.tile != TILE_OLD) {
+      if constexpr (SWI)
+        launch_tile<GtBig, GT_SWIGLU>(p, w, si, sb, x, bias, y, nullptr, in_f, out_f, 2 * out_f, n,
+                                      accum, GtRope{});
+      else if (p.tile == TILE_BIG)
+        launch_tile<GtBig, GT_PLAIN>(p, w, si, sb, x, bias, y, ws, in_f, out_f, out_f, n, accum,
+                                     GtRope{});
+      else
+        launch_tile<GtSmall, GT_PLAIN>(p, w, si, sb, x, bias, y, ws, in_f, out_f, out_f, n, accum,
+                                       GtRope{});
+      return;
+    }
+  }
   set_lds_attr<HIER, SWI>();
   if constexpr (HIER) {
     if (p.wide) {
       if (p.nwv == 4)
         gemm_wide_kernel<HIER, SWI, 4><<<p.grid, GwShape<4>::THREADS, GwShape<4>::LDS, WST_STREAM>>>(
             w, (const uint8_t *)si, (const uint32_t *)sb, (const uint16_t *)x,
-            (const uint16_t *)bias, (float *)y, ws, in_f, out_f, n, accum, p.gps, GwRope{});
+            (const uint16_t *)bias, (float *)y, ws, in_f, out_f, n, accum, p.gps);
       else
         gemm_wide_kernel<HIER, SWI, 8><<<p.grid, GwShape<8>::THREADS, GwShape<8>::LDS, WST_STREAM>>>(
             w, (const uint8_t *)si, (const uint32_t *)sb, (const uint16_t *)x,
-            (const uint16_t *)bias, (float *)y, ws, in_f, out_f, n, accum, p.gps, GwRope{});
+            (const uint16_t *)bias, (float *)y, ws, in_f, out_f, n, accum, p.gps);
       return;
     }
   }
@@ -1244,7 +1228,7 @@ void launch_gemm(const GemmPlan &p, const void *w, const void *si, const void *s
 wst_status_t gemm_to_scratch(const void *w, const void *si, const void *sb, const void *x,
                              int in_f, int out_f, int n, float **ws_out, int *splits_out,
                              int plan_n = 0) {
-  const GemmPlan p = plan_gemm(in_f, out_f, n, true, 0, false, plan_n);
+  const GemmPlan p = plan_gemm(in_f, out_f, n, true, 0, false, plan_n, si);
   float *ws = (float *)wst_static_scratch(WST_SCRATCH_GEMM, (size_t)p.splits * n * out_f * 4);
   if (!ws) return WST_ERR_OOM;
   launch_gemm<true, false>(p, w, si, sb, x, nullptr, nullptr, ws, in_f, out_f, n, 0);
@@ -1260,7 +1244,8 @@ wst_status_t wst_gemm_mfma(bool hier, const void *w, const void *si, const void 
                            const void *x, const void *bias, void *y, int32_t in_f, int32_t out_f,
                            int32_t n, int32_t accum, float *ws_ext, size_t ws_cap,
                            int32_t plan_n) {
-  const GemmPlan p = plan_gemm(in_f, out_f, n, hier, 0, false, plan_n);
+  const GemmPlan p = plan_gemm(in_f, out_f, n, hier, 0, false, plan_n, si,
+                               ws_ext ? ws_cap : (size_t)256 << 20);
   const int splits = p.splits;
   float *ws = nullptr;
   if (splits > 1) {
@@ -1315,10 +1300,14 @@ extern "C" wst_status_t wst_gemm_hier_swiglu_chunks(const void *qw, const void *
   if (st != WST_OK) return st;
   WST_REQUIRE(act, "wst_gemm_hier_swiglu_chunk: null pointer");
   // Never split: a tile pairs BM/2 gate rows with the matching up rows.
-  GemmPlan p = plan_gemm(in_f, inter, n, true, 2 * inter, true, plan_n);
-  p.splits = 1;
-  p.gps = in_f / HGROUP;
-  p.grid = dim3((inter + p.bm / 2 - 1) / (p.bm / 2), (n + p.bn - 1) / p.bn, 1);
+  GemmPlan p = plan_gemm(in_f, inter, n, true, 2 * inter, true, plan_n, si);
+  if (p.tile != TILE_OLD) {
+    p.grid = dim3((unsigned)(((inter + p.bm / 2 - 1) / (p.bm / 2)) * ((n + p.bn - 1) / p.bn)), 1, 1);
+  } else {
+    p.splits = 1;
+    p.gps = in_f / HGROUP;
+    p.grid = dim3((inter + p.bm / 2 - 1) / (p.bm / 2), (n + p.bn - 1) / p.bn, 1);
+  }
   launch_gemm<true, true>(p, qw, si, sb, x, nullptr, act, nullptr, in_f, inter, n, 0);
   WST_TRY_KERNEL("wst_gemm_hier_swiglu_chunk");
   return WST_OK;
@@ -1407,26 +1396,24 @@ extern "C" wst_status_t wst_gemm_hier_rope_chunks(const void *qw, const void *si
               "wst_gemm_hier_rope_chunk: null pointer");
   WST_REQUIRE(max_seq > 0 && pos0 >= 0 && pos0 + n <= max_seq,
               "wst_gemm_hier_rope_chunk: chunk does not fit the cache");
-  // head_dim 64 on unsplit 256-token wide tiles (a batched prefill of the
-  // 0.5B shape): each tile is one head, and its epilogue applies the norm,
-  // the rotation and the cache append itself, in the reduce kernel's
-  // arithmetic; no partials, no second launch.
+  // Unsplit big tiles at head_dim 64 or 128: a wave holds whole rotation pairs
+  // (at 64 a whole head), so the epilogue applies the norm, the rotation and
+  // the cache append itself, in the reduce kernel's arithmetic; no partials, no
+  // second launch. The QK-norm of a 128-wide head would sum over two waves:
+  // those take the reduce kernel.
   {
-    const GemmPlan p = plan_gemm(in_f, out_f, n, true, 0, false, plan_n);
-    if (p.wide && p.nwv == 8 && p.splits == 1 && head_dim == GW_ROPE_HD && rope_epilogue_on()) {
-      static bool attr = false;
-      if (!attr) {
-        (void)hipFuncSetAttribute((const void *)gemm_wide_kernel<true, false, 8, true>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, GwShape<8>::LDS);
-        attr = true;
-      }
-      const GwRope re{(uint16_t *)k_cache, (uint16_t *)v_cache, (const float *)cos_tab,
+    const GemmPlan p = plan_gemm(in_f, out_f, n, true, 0, false, plan_n, si);
+    if (p.tile == TILE_BIG && p.splits == 1 && rope_epilogue_on() &&
+        (head_dim == 64 || (head_dim == 128 && !q_norm_w && !k_norm_w))) {
+      const GtRope re{(uint16_t *)k_cache, (uint16_t *)v_cache, (const float *)cos_tab,
                       (const float *)sin_tab, (const uint16_t *)q_norm_w,
                       (const uint16_t *)k_norm_w, n_q, n_kv, pos0, max_seq, eps};
-      gemm_wide_kernel<true, false, 8, true><<<p.grid, GwShape<8>::THREADS, GwShape<8>::LDS,
-                                               WST_STREAM>>>(
-          qw, (const uint8_t *)si, (const uint32_t *)sb, (const uint16_t *)x,
-          (const uint16_t *)bias, (float *)qkv, nullptr, in_f, out_f, n, 0, p.gps, re);
+      if (head_dim == 64)
+        launch_tile<GtBig, GT_ROPE64>(p, qw, si, sb, x, bias, qkv, nullptr, in_f, out_f, out_f, n,
+                                      0, re);
+      else
+        launch_tile<GtBig, GT_ROPE128>(p, qw, si, sb, x, bias, qkv, nullptr, in_f, out_f, out_f, n,
+                                       0, re);
       WST_TRY_KERNEL("wst_gemm_hier_rope_chunk");
       return WST_OK;
     }
