@@ -38,6 +38,7 @@
 #include "gemm_tile.hpp"
 
 #include <mutex>
+#include <type_traits>
 
 #define HGROUP 32
 #define GM_BM 64
@@ -1011,11 +1012,16 @@ void set_lds_attr() {
   }
 }
 
-// Register-dequantising tiles (gemm_tile.hpp): 256 rows x 128 tokens in four
-// waves of 64 x 128, and 128 rows x 128 tokens in eight waves of 32 x 64.
+// Register-dequantising tiles (gemm_tile.hpp), four waves each: 256 rows x 128
+// tokens (waves of 64 x 128), 128 rows x 64 tokens (32 x 64) and 128 rows x 32
+// tokens (32 x 32); the SwiGLU forms pair a gate and an up fragment in every
+// wave, so their small tiles are 256 weight rows too.
 using GtBig = GtShape<4, 1, 2, 4>;
-using GtSmall = GtShape<4, 2, 1, 2>;
-enum GemmTile { TILE_OLD = 0, TILE_BIG = 1, TILE_SMALL = 2 };
+using GtMid = GtShape<4, 1, 1, 2>;
+using GtLow = GtShape<4, 1, 1, 1>;
+using GtMidSwi = GtShape<4, 1, 2, 2>;
+using GtLowSwi = GtShape<4, 1, 2, 1>;
+enum GemmTile { TILE_OLD = 0, TILE_BIG = 1, TILE_MID = 2, TILE_LOW = 3 };
 
 struct GemmPlan {
   int tile;  // GemmTile; TILE_OLD: the LDS tiles (wide or not, below)
@@ -1055,36 +1061,51 @@ bool tile_ok(const void *si, int in_f, int out_f, int rows, int n) {
          (size_t)n * out_f * 4 < lim && out_f <= (1 << 20);
 }
 
-// Tile and K split by the time the most loaded CU takes: blocks per CU x steps
-// per block x the tile's step time, plus the tile's fixed part (launch,
-// first loads, stores) and the partials' traffic. Step and fixed times
-// measured over 896..18944-column rows and 256..4096 tokens: big 1.8 us and
-// 12 us, small 1.45 us and 7 us (two blocks on a CU take twice as long as one:
-// they share the matrix cores and the VALU), partials 4 TB/s. A split's
-// partials stay below max_part bytes.
-void plan_tile(GemmPlan &p, int in_f, int out_f, int rows, int pn, int n, bool may_split,
-               bool small_ok, size_t max_part) {
+// What a block of a tile costs: a step alone on its CU (lat), a step's share of
+// a CU that several blocks keep busy (thr), and launch, first loads and stores
+// (fixed), in us. Measured over rows of 896..18944 columns and 5..4096 tokens.
+struct TileCost {
+  int bm, bn;
+  float lat, thr, fixed;
+};
+constexpr TileCost TILE_COST[2][3] = {
+    {{GtBig::BM, GtBig::BN, 1.8f, 1.9f, 8.0f},
+     {GtMid::BM, GtMid::BN, 0.7f, 0.75f, 4.5f},
+     {GtLow::BM, GtLow::BN, 0.8f, 0.55f, 4.0f}},
+    {{GtBig::BM, GtBig::BN, 1.8f, 1.9f, 6.0f},
+     {GtMidSwi::BM, GtMidSwi::BN, 1.27f, 1.2f, 4.5f},
+     {GtLowSwi::BM, GtLowSwi::BN, 1.05f, 0.95f, 4.5f}}};
+
+// The tile and K split of the least estimated time: steps a block x what a
+// step takes with the blocks the fullest CU holds, the tile's fixed part, and
+// for a split the reduce launch and the partials' way out and back (4 TB/s).
+// The partials stay below max_part bytes; the SwiGLU form never splits. A
+// token's bits depend on the split only, not on the tile.
+// Where it lies, measured in us (big / mid / low): 896 -> 1152 x 4096 tokens
+// 20.9 / 18.7 / -; 7B gate|up x 232 101 / 101 / 130, x 30 53 / 38 / 33;
+// 896 -> 151936 x 30 49 / 28 / 22; 3584 -> 4608 x 30 unsplit low 29, split 7
+// ways 9 with its reduce.
+void plan_tile(GemmPlan &p, int in_f, int out_f, int rows, int pn, int n, bool swi,
+               size_t max_part) {
   const int steps = in_f / GT_KC, cus = wst_cu_count();
   float best = 0.0f;
   p.tile = TILE_OLD;
-  for (int t = TILE_BIG; t <= (small_ok ? TILE_SMALL : TILE_BIG); ++t) {
-    const int bm = t == TILE_BIG ? GtBig::BM : GtSmall::BM;
-    const int bn = t == TILE_BIG ? GtBig::BN : GtSmall::BN;
-    const float step_us = t == TILE_BIG ? 1.8f : 1.45f, fixed_us = t == TILE_BIG ? 12.0f : 7.0f;
-    const int tiles = ((rows + bm - 1) / bm) * ((pn + bn - 1) / bn);
-    for (int want = 1; want <= (may_split ? GM_MAXSPLIT : 1) && want <= steps; ++want) {
+  for (int t = TILE_BIG; t <= TILE_LOW; ++t) {
+    const TileCost &c = TILE_COST[swi][t - 1];
+    const int tiles = ((rows + c.bm - 1) / c.bm) * ((pn + c.bn - 1) / c.bn);
+    for (int want = 1; want <= (swi ? 1 : GM_MAXSPLIT) && want <= steps; ++want) {
       const int sps = (steps + want - 1) / want, splits = (steps + sps - 1) / sps;
-      const size_t part = (size_t)splits * n * out_f * 4;
-      if (splits > 1 && part > max_part) break;
+      if (splits > 1 && (size_t)splits * n * out_f * 4 > max_part) break;
       if (gemm_split_cap() > 0 && splits > gemm_split_cap()) break;
-      const float us = (float)((tiles * splits + cus - 1) / cus) * (float)sps * step_us + fixed_us +
-                       (splits > 1 ? 3.0f + (float)splits * (float)pn * (float)out_f * 8.0f / 4.0e6f
-                                   : 0.0f);
+      const float held = (float)((tiles * splits + cus - 1) / cus);
+      const float step = c.thr * held > c.lat ? c.thr * held : c.lat;
+      float us = (float)sps * step + c.fixed;
+      if (splits > 1) us += 3.5f + (float)splits * (float)pn * (float)out_f * 8.0f / 4.0e6f;
       if (p.tile == TILE_OLD || us < best) {
         best = us;
         p.tile = t;
-        p.bm = bm;
-        p.bn = bn;
+        p.bm = c.bm;
+        p.bn = c.bn;
         p.splits = splits;
         p.gps = sps;  // steps of GT_KC columns
       }
@@ -1114,7 +1135,7 @@ GemmPlan plan_gemm(int in_f, int out_f, int n, bool hier = true, int rows = 0, b
   if (rows <= 0) rows = out_f;
   const int pn = plan_n > 0 && plan_n < n ? plan_n : n;
   if (hier && tile_ok(si, in_f, out_f, rows, n)) {
-    plan_tile(p, in_f, out_f, rows, pn, n, !swi, !swi, max_part);
+    plan_tile(p, in_f, out_f, rows, pn, n, swi, max_part);
     p.wide = false;
     p.nwv = 0;
     p.kg = 0;
@@ -1192,15 +1213,16 @@ void launch_gemm(const GemmPlan &p, const void *w, const void *si, const void *s
                  const void *bias, void *y, float *ws, int in_f, int out_f, int n, int accum) {
   if constexpr (HIER) {
     if (p.tile != TILE_OLD) {
-      if constexpr (SWI)
-        launch_tile<GtBig, GT_SWIGLU>(p, w, si, sb, x, bias, y, nullptr, in_f, out_f, 2 * out_f, n,
-                                      accum, GtRope{});
-      else if (p.tile == TILE_BIG)
-        launch_tile<GtBig, GT_PLAIN>(p, w, si, sb, x, bias, y, ws, in_f, out_f, out_f, n, accum,
-                                     GtRope{});
-      else
-        launch_tile<GtSmall, GT_PLAIN>(p, w, si, sb, x, bias, y, ws, in_f, out_f, out_f, n, accum,
-                                       GtRope{});
+      constexpr int E = SWI ? GT_SWIGLU : GT_PLAIN;
+      using Mid = std::conditional_t<SWI, GtMidSwi, GtMid>;
+      using Low = std::conditional_t<SWI, GtLowSwi, GtLow>;
+      auto go = [&](auto shape) {
+        launch_tile<decltype(shape), E>(p, w, si, sb, x, bias, y, ws, in_f, out_f,
+                                        SWI ? 2 * out_f : out_f, n, accum, GtRope{});
+      };
+      if (p.tile == TILE_BIG) go(GtBig{});
+      else if (p.tile == TILE_MID) go(Mid{});
+      else go(Low{});
       return;
     }
   }
