@@ -61,7 +61,7 @@ struct wse_engine {
   void *c_tokens = nullptr, *c_x = nullptr, *c_h = nullptr, *c_qkv = nullptr, *c_attn = nullptr,
        *c_act = nullptr;
   void *c_logits = nullptr, *c_picks = nullptr;  // the chunk head's, on first use
-  // Buffers of a prefill whose full chunks share their launches (b_cap tokens).
+  // Buffers of a prefill whose chunks share their launches (b_cap tokens).
   int b_cap = 0;
   void *b_tokens = nullptr, *b_x = nullptr, *b_h = nullptr, *b_qkv = nullptr,
        *b_attn = nullptr, *b_act = nullptr;
@@ -1011,8 +1011,9 @@ static wst_status_t ensure_batch(wse_engine *e, int n) {
   return WST_OK;
 }
 
-// The full chunks of a chunked prefill go through each layer together
-// (chunk_pass with n > width), planned for the whole launch (1, the default);
+// The chunks of a chunked prefill go through each layer together (chunk_pass
+// with n > width), planned for the whole launch (1, the default: a shorter last
+// chunk goes along, 7B prefill of 1000 tokens 20.9 -> 17.0 ms);
 // WSE_CHUNK_BATCH=chunk keeps one chunk's plan per launch (bit-identical to
 // the chunk-by-chunk pass); WSE_CHUNK_BATCH=0 runs the chunks one by one.
 enum BatchMode { BATCH_OFF, BATCH_WHOLE, BATCH_CHUNK_PLAN };
@@ -1083,13 +1084,16 @@ wst_status_t wse_engine_prefill(wse_engine_t *e, const int32_t *ids, int32_t n, 
     TRY(ensure_chunk(e));
     const int w = e->chunk_width;
     int s = 0;
-    const int full = n / w * w;  // the full chunks (a shorter last chunk keeps its own plan)
     const BatchMode mode = chunk_batch_mode();
-    if (mode != BATCH_OFF && full >= 2 * w) {
-      TRY(ensure_batch(e, full));
+    // One plan for the whole launch takes the shorter last chunk along (the
+    // weights are read once for all the prompt's tokens); one chunk's plan
+    // leaves it its own.
+    const int batch = mode == BATCH_CHUNK_PLAN ? n / w * w : n;
+    if (mode != BATCH_OFF && (batch >= 2 * w || (mode == BATCH_WHOLE && n > w))) {
+      TRY(ensure_batch(e, (batch + w - 1) / w * w));
       const ChunkBufs b{e->b_tokens, e->b_x, e->b_h, e->b_qkv, e->b_attn, e->b_act};
-      TRY(chunk_pass(e, ids, full, full == n, w, mode == BATCH_CHUNK_PLAN ? w : 0, b));
-      s = full;
+      TRY(chunk_pass(e, ids, batch, batch == n, w, mode == BATCH_CHUNK_PLAN ? w : 0, b));
+      s = batch;
     }
     for (; s < n; s += w) {
       const int k = n - s < w ? n - s : w;
