@@ -1078,7 +1078,8 @@ constexpr TileCost TILE_COST[2][3] = {
 
 // The tile and K split of the least estimated time: steps a block x what a
 // step takes with the blocks the fullest CU holds, the tile's fixed part, and
-// for a split the reduce launch and the partials' way out and back (4 TB/s).
+// for a split a reduce launch and each further partial's way out and back (4
+// TB/s; the residual and qkv forms write one partial and reduce it anyway).
 // The partials stay below max_part bytes; the SwiGLU form never splits. A
 // token's bits depend on the split only, not on the tile.
 // Where it lies, measured in us (big / mid / low): 896 -> 1152 x 4096 tokens
@@ -1100,7 +1101,7 @@ void plan_tile(GemmPlan &p, int in_f, int out_f, int rows, int pn, int n, bool s
       const float held = (float)((tiles * splits + cus - 1) / cus);
       const float step = c.thr * held > c.lat ? c.thr * held : c.lat;
       float us = (float)sps * step + c.fixed;
-      if (splits > 1) us += 3.5f + (float)splits * (float)pn * (float)out_f * 8.0f / 4.0e6f;
+      if (splits > 1) us += 3.5f + (float)(splits - 1) * (float)pn * (float)out_f * 8.0f / 4.0e6f;
       if (p.tile == TILE_OLD || us < best) {
         best = us;
         p.tile = t;
@@ -1418,24 +1419,34 @@ extern "C" wst_status_t wst_gemm_hier_rope_chunks(const void *qw, const void *si
               "wst_gemm_hier_rope_chunk: null pointer");
   WST_REQUIRE(max_seq > 0 && pos0 >= 0 && pos0 + n <= max_seq,
               "wst_gemm_hier_rope_chunk: chunk does not fit the cache");
-  // Unsplit big tiles at head_dim 64 or 128: a wave holds whole rotation pairs
-  // (at 64 a whole head), so the epilogue applies the norm, the rotation and
-  // the cache append itself, in the reduce kernel's arithmetic; no partials, no
-  // second launch. The QK-norm of a 128-wide head would sum over two waves:
-  // those take the reduce kernel.
+  // Unsplit at head_dim 64 or 128: the tiles of two fragments a wave hold whole
+  // rotation pairs (at 64 a whole head), so their epilogue applies the norm,
+  // the rotation and the cache append itself, in the reduce kernel's
+  // arithmetic; no partials, no second launch (0.5B qkv over 4096 tokens 18.7
+  // + 21.1 us in two launches, 7B over 1000 tokens 58 + 18). Unsplit tiles all
+  // give the same bits, so their choice here is free. The QK-norm of a
+  // 128-wide head would sum over two waves: those take the reduce kernel.
   {
-    const GemmPlan p = plan_gemm(in_f, out_f, n, true, 0, false, plan_n, si);
-    if (p.tile == TILE_BIG && p.splits == 1 && rope_epilogue_on() &&
-        (head_dim == 64 || (head_dim == 128 && !q_norm_w && !k_norm_w))) {
+    GemmPlan p = plan_gemm(in_f, out_f, n, true, 0, false, plan_n, si);
+    if (p.tile != TILE_OLD && p.splits == 1 && rope_epilogue_on() &&
+        (head_dim == 64 || (head_dim == 128 && !q_norm_w && !k_norm_w)) &&
+        (size_t)max_seq * head_dim * 2 < ((size_t)1 << 31)) {
+      plan_tile(p, in_f, out_f, out_f, n, n, true, 0);
+      p.grid = dim3((unsigned)(((out_f + p.bm - 1) / p.bm) * ((n + p.bn - 1) / p.bn)), 1, 1);
       const GtRope re{(uint16_t *)k_cache, (uint16_t *)v_cache, (const float *)cos_tab,
                       (const float *)sin_tab, (const uint16_t *)q_norm_w,
                       (const uint16_t *)k_norm_w, n_q, n_kv, pos0, max_seq, eps};
-      if (head_dim == 64)
-        launch_tile<GtBig, GT_ROPE64>(p, qw, si, sb, x, bias, qkv, nullptr, in_f, out_f, out_f, n,
-                                      0, re);
-      else
-        launch_tile<GtBig, GT_ROPE128>(p, qw, si, sb, x, bias, qkv, nullptr, in_f, out_f, out_f, n,
-                                       0, re);
+      auto go = [&](auto shape) {
+        if (head_dim == 64)
+          launch_tile<decltype(shape), GT_ROPE64>(p, qw, si, sb, x, bias, qkv, nullptr, in_f,
+                                                  out_f, out_f, n, 0, re);
+        else
+          launch_tile<decltype(shape), GT_ROPE128>(p, qw, si, sb, x, bias, qkv, nullptr, in_f,
+                                                   out_f, out_f, n, 0, re);
+      };
+      if (p.tile == TILE_BIG) go(GtBig{});
+      else if (p.tile == TILE_MID) go(GtMidSwi{});
+      else go(GtLowSwi{});
       WST_TRY_KERNEL("wst_gemm_hier_rope_chunk");
       return WST_OK;
     }

@@ -303,48 +303,79 @@ __global__ __launch_bounds__(S::THREADS, S::MT * S::NT > 8 ? 1 : 2) void gemm_ti
     const int h = base / HD, jj = EPI == GT_ROPE64 ? l32 : (wm & 1) * 32 + l32;
     const float b1 = bias ? h2f(bias[base + jj]) : 0.0f;
     const float b2 = bias ? h2f(bias[base + jj + HALF]) : 0.0f;
-    const bool is_q = h < re.n_q, is_v = h >= re.n_q + re.n_kv;
+    const bool is_q = h < re.n_q, is_v = h >= re.n_q + re.n_kv;  // uniform in the wave
     const uint16_t *g = is_v ? nullptr : is_q ? re.q_norm_w : re.k_norm_w;
     const float g1 = g ? h2f(g[jj]) : 0.0f, g2 = g ? h2f(g[jj + HALF]) : 0.0f;
     const int kvh = is_v ? h - re.n_q - re.n_kv : h - re.n_q;
-    uint16_t *cache = is_v ? re.v_cache : re.k_cache;
+    // Rows of y and of the head's cache by buffer offsets: a token past n gets
+    // an offset past the range and is dropped.
+    const uint32_t tb = (uint32_t)out_f * 4u;
+    const __amdgpu_buffer_rsrc_t yrs =
+        __builtin_amdgcn_make_buffer_rsrc((void *)y, 0, (int)((uint32_t)n * tb), 0x00020000);
+    const uint32_t yoff = tok0 * tb + (uint32_t)(base + jj) * 4u;
+    const size_t head0 = (size_t)(is_q ? 0 : kvh) * re.max_seq + re.pos0;
+    const __amdgpu_buffer_rsrc_t crs = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)((is_v ? re.v_cache : re.k_cache) + head0 * HD), 0,
+        (int)((uint32_t)n * (uint32_t)(HD * 2)), 0x00020000);
+    const uint32_t coff = tok0 * (uint32_t)(HD * 2) + (uint32_t)jj * 2u;
+    const uint32_t rot = (uint32_t)(n * HALF * 4);  // the tokens' rows of the rotation tables
+    const __amdgpu_buffer_rsrc_t cosr = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(re.cos_tab + (size_t)re.pos0 * HALF), 0, (int)rot, 0x00020000);
+    const __amdgpu_buffer_rsrc_t sinr = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(re.sin_tab + (size_t)re.pos0 * HALF), 0, (int)rot, 0x00020000);
+    const uint32_t roff = tok0 * (uint32_t)(HALF * 4) + (uint32_t)jj * 4u;
+    auto store_f = [&](float v, uint32_t off) {
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), yrs, off, 0, 0);
+    };
+    if (is_v) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const uint32_t dt = (uint32_t)(32 * t + 8 * (r >> 2) + (r & 3));
+          float x1 = acc[0][t][r], x2 = acc[1][t][r];
+          if (bias) {
+            x1 += b1;
+            x2 += b2;
+          }
+          store_f(x1, yoff + dt * tb);
+          store_f(x2, yoff + dt * tb + HALF * 4u);
+          __builtin_amdgcn_raw_buffer_store_b16(f2h(x1), crs, coff + dt * (HD * 2u), 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b16(f2h(x2), crs, coff + dt * (HD * 2u) + HALF * 2u, 0, 0);
+        }
+      return;
+    }
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      float c[16], sn[16];
+      uint32_t c[16], sn[16];
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int tok = (int)tok0 + 32 * t + 8 * (r >> 2) + (r & 3);
-        const int pos = min(re.pos0 + min(tok, n - 1), re.max_seq - 1);
-        c[r] = re.cos_tab[(size_t)pos * HALF + jj];
-        sn[r] = re.sin_tab[(size_t)pos * HALF + jj];
+        const uint32_t dt = (uint32_t)(32 * t + 8 * (r >> 2) + (r & 3));
+        c[r] = __builtin_amdgcn_raw_buffer_load_b32(cosr, roff + dt * (HALF * 4u), 0, 0);
+        sn[r] = __builtin_amdgcn_raw_buffer_load_b32(sinr, roff + dt * (HALF * 4u), 0, 0);
       }
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int tok = (int)tok0 + 32 * t + 8 * (r >> 2) + (r & 3);
+        const uint32_t dt = (uint32_t)(32 * t + 8 * (r >> 2) + (r & 3));
         float x1 = acc[0][t][r], x2 = acc[1][t][r];
         if (bias) {
           x1 += b1;
           x2 += b2;
         }
-        const float k1 = x1, k2 = x2;  // k and v rows keep the value as computed
+        const float k1 = x1, k2 = x2;  // a k row keeps the value as computed
         if (EPI == GT_ROPE64 && g) {
           const float ss = half_wave_sum(fmaf(x1, x1, x2 * x2));
           const float sc = 1.0f / sqrtf(ss / (float)HD + re.eps);
           x1 = x1 * sc * g1;
           x2 = x2 * sc * g2;
         }
-        const float lo = is_v ? k1 : rope_lo(x1, x2, c[r], sn[r]);
-        const float hi = is_v ? k2 : rope_hi(x1, x2, c[r], sn[r]);
-        if (tok < n) {
-          float *row = y + (size_t)tok * out_f + base + jj;
-          row[0] = is_q ? lo : k1;
-          row[HALF] = is_q ? hi : k2;
-          if (!is_q) {
-            const int pos = min(re.pos0 + tok, re.max_seq - 1);
-            uint16_t *slot = cache + ((size_t)kvh * re.max_seq + pos) * HD + jj;
-            slot[0] = f2h(lo);
-            slot[HALF] = f2h(hi);
-          }
+        const float cv = __builtin_bit_cast(float, c[r]), sv = __builtin_bit_cast(float, sn[r]);
+        const float lo = rope_lo(x1, x2, cv, sv), hi = rope_hi(x1, x2, cv, sv);
+        store_f(is_q ? lo : k1, yoff + dt * tb);
+        store_f(is_q ? hi : k2, yoff + dt * tb + HALF * 4u);
+        if (!is_q) {
+          __builtin_amdgcn_raw_buffer_store_b16(f2h(lo), crs, coff + dt * (HD * 2u), 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b16(f2h(hi), crs, coff + dt * (HD * 2u) + HALF * 2u, 0, 0);
         }
       }
     }
