@@ -212,6 +212,14 @@ wst_status_t wst_gemm_hier_rope_chunks(const void *qw, const void *si, const voi
                                        int32_t max_seq, const void *q_norm_w,
                                        const void *k_norm_w, float eps, int32_t plan_n);
 
+/* wst_attn_chunk over n tokens that hold several chunks, each token with the
+ * bits a call of plan_n tokens gives it (the planned count picks how the keys
+ * are split into partial sums); plan_n = 0 or n is wst_attn_chunk. */
+wst_status_t wst_attn_chunks(const void *qkv, const void *k_cache, const void *v_cache,
+                             void *out, int32_t n_q, int32_t n_kv, int32_t head_dim,
+                             int32_t pos0, int32_t n, int32_t max_seq, float scale,
+                             int32_t plan_n);
+
 /* ------------------------------------------------------------ measurement */
 
 /* One launch of the library's streaming-read kernel (16-byte nontemporal

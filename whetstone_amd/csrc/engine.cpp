@@ -953,8 +953,8 @@ static wst_status_t chunk_pass(wse_engine *e, const int32_t *ids, int n, bool wa
                                e->sin_tab, nq, nkv, hd, pos0, n, e->max_seq, L.q_norm, L.k_norm,
                                eps));
     }
-    TRY(wst_attn_chunk(b.qkv, e->kc[(size_t)l], e->vc[(size_t)l], b.attn, nq, nkv, hd, pos0, n,
-                       e->max_seq, scale));
+    TRY(wst_attn_chunks(b.qkv, e->kc[(size_t)l], e->vc[(size_t)l], b.attn, nq, nkv, hd, pos0, n,
+                        e->max_seq, scale, pn));
     TRY(wst_gemm_hier_norm_chunks(L.o.qw, L.o.si, L.o.sb, b.attn, nullptr, b.x, nq * hd, H, n, 1,
                                   L.post_norm, eps, b.h, pn));
     TRY(wst_gemm_hier_swiglu_chunks(L.gate_up.qw, L.gate_up.si, L.gate_up.sb, b.h, b.act, H, I,

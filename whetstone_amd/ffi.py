@@ -124,6 +124,7 @@ ABI = {
     "wst_rmsnorm_chunk": (I32, [P, P, P, I32, I32, F32]),
     "wst_rope_cache_chunk": (I32, [P, P, P, P, P, I32, I32, I32, I32, I32, I32, P, P, F32]),
     "wst_attn_chunk": (I32, [P, P, P, P, I32, I32, I32, I32, I32, I32, F32]),
+    "wst_attn_chunks": (I32, [P, P, P, P, I32, I32, I32, I32, I32, I32, F32, I32]),
     "wst_swiglu_chunk": (I32, [P, P, I32, I32]),
     "wst_embed_fp16_chunk": (I32, [P, P, P, I32, I32, I32]),
     "wst_embed_int4_hier_chunk": (I32, [P, P, P, P, P, I32, I32, I32]),
