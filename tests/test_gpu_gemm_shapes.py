@@ -47,14 +47,18 @@ def test_gemm_odd_group_counts(orc, wk, in_f, out_f, n, accum):
     _check(y.numpy().astype(np.float64).reshape(n, out_f), x, w, ref)
 
 
-# rows of whole 128-column steps: one step, an odd and an even count of them;
-# one row, a row tile's edge and one past it; one token, a token tile's edge
+# rows of 128-column steps: one step, an odd and an even count of them; one row, a row tile's edge and one past it; one token, a token tile's edge
 # and one past it; K split (long rows) with and without the accumulate
 @pytest.mark.parametrize("in_f,out_f,n,accum", [(128, 1, 1, False), (256, 256, 128, True),
                                                 (384, 257, 129, False), (896, 127, 127, True),
                                                 (1152, 130, 70, False), (4864, 896, 256, True),
-                                                (3584, 1056, 1000, False), (9216, 33, 200, True)])
-def test_gemm_whole_step_rows(orc, wk, in_f, out_f, n, accum):
+                                                (3584, 1056, 1000, False), (9216, 33, 200, True),
+                                                # rows that end in half a step: a step and a half, split
+                                                # and unsplit, each token tile
+                                                (192, 1, 1, False), (192, 300, 33, True),
+                                                (960, 257, 65, False), (4928, 96, 7, True),
+                                                (1216, 9000, 600, False)])
+def test_gemm_step_rows(orc, wk, in_f, out_f, n, accum):
     print(f"gemm {in_f} -> {out_f}, {n} tokens", flush=True)
     lin, w, x, xd, bias, bd = _operands(orc, wk, in_f, out_f, n, 62)
     y0 = orc.fixture_normal(62, 4, (n + 1) * out_f, 1.0)
@@ -70,8 +74,8 @@ def test_gemm_whole_step_rows(orc, wk, in_f, out_f, n, accum):
 
 
 @pytest.mark.parametrize("in_f,inter,n", [(128, 1, 1), (256, 128, 128), (896, 161, 129),
-                                          (384, 700, 300)])
-def test_gemm_swiglu_whole_step_rows(orc, wk, in_f, inter, n):
+                                          (384, 700, 300), (192, 100, 40), (320, 4000, 300)])
+def test_gemm_swiglu_step_rows(orc, wk, in_f, inter, n):
     print(f"gate|up {in_f} -> {inter}, {n} tokens", flush=True)
     lin, w, x, xd, _, _ = _operands(orc, wk, in_f, 2 * inter, n, 63)
     act = wk.DeviceBuffer.from_array(np.full((n + 1) * inter, 7.0, np.float16))
@@ -91,12 +95,16 @@ def test_gemm_swiglu_whole_step_rows(orc, wk, in_f, inter, n):
 
 
 @pytest.mark.parametrize("in_f,n_q,n_kv,hd,pos0,n,qk", [(3584, 28, 4, 128, 5, 2049, False),
-                                                        (896, 14, 2, 64, 3, 4000, True)])
+                                                        (896, 14, 2, 64, 3, 4000, True),
+                                                        (192, 14, 2, 64, 0, 20, True),
+                                                        (192, 14, 2, 64, 7, 130, False),
+                                                        (256, 8, 2, 128, 0, 20, False),
+                                                        (256, 28, 4, 128, 1, 700, False)])
 def test_gemm_rope_epilogue_equals_gemm_then_rope_cache(orc, wk, in_f, n_q, n_kv, hd, pos0, n, qk):
-    """Enough tokens that the projection runs unsplit on the big tiles, whose
-    epilogue rotates and appends: against the GEMM then wst_rope_cache_chunk,
-    bit for bit, at both head sizes (the last token tile ragged, the cache
-    ending at the last token)."""
+    """Shapes whose projection runs unsplit, so that the tiles' epilogue rotates
+    and appends: against the GEMM then wst_rope_cache_chunk, bit for bit, at
+    both head sizes and each token tile (the last one ragged, the cache ending
+    at the last token)."""
     print(f"rope epilogue hd {hd}, {n} tokens", flush=True)
     out_f, max_seq = (n_q + 2 * n_kv) * hd, pos0 + n
     lin = wk.QuantLinearHier(*(wk.DeviceBuffer(k, t) for k, t in (

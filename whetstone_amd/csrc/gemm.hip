@@ -1052,11 +1052,12 @@ static int gemm_bn_override() {
   return v;
 }
 
-// The register-dequantising tiles take int4-hier rows of whole 128-column
-// steps with 4-byte aligned index bytes, within their 32-bit offsets.
+// The register-dequantising tiles take int4-hier rows of 128 columns or more in
+// whole 64-column halves of a step, with 4-byte aligned index bytes, within
+// their 32-bit offsets.
 bool tile_ok(const void *si, int in_f, int out_f, int rows, int n) {
   const size_t lim = (size_t)1 << 31;
-  return gemm_tiles_mode() == 1 && in_f % GT_KC == 0 && !((uintptr_t)si & 3u) &&
+  return gemm_tiles_mode() == 1 && in_f % 64 == 0 && in_f >= GT_KC && !((uintptr_t)si & 3u) &&
          (size_t)n * in_f * 2 < lim && (size_t)rows * (in_f / 2) < lim &&
          (size_t)n * out_f * 4 < lim && out_f <= (1 << 20);
 }
@@ -1088,7 +1089,7 @@ constexpr TileCost TILE_COST[2][3] = {
 // ways 9 with its reduce.
 void plan_tile(GemmPlan &p, int in_f, int out_f, int rows, int pn, int n, bool swi,
                size_t max_part) {
-  const int steps = in_f / GT_KC, cus = wst_cu_count();
+  const int steps = (in_f + GT_KC - 1) / GT_KC, cus = wst_cu_count();
   float best = 0.0f;
   p.tile = TILE_OLD;
   for (int t = TILE_BIG; t <= TILE_LOW; ++t) {
@@ -1188,13 +1189,13 @@ GemmPlan plan_gemm(int in_f, int out_f, int n, bool hier = true, int rows = 0, b
   return p;
 }
 
-template <class S, int EPI>
-void launch_tile(const GemmPlan &p, const void *w, const void *si, const void *sb, const void *x,
+template <class S, int EPI, bool TAIL>
+void launch_tile_t(const GemmPlan &p, const void *w, const void *si, const void *sb, const void *x,
                  const void *bias, void *y, float *ws, int in_f, int out_f, int rows, int n,
                  int accum, const GtRope &re) {
   static bool attr = false;
   if (!attr) {
-    (void)hipFuncSetAttribute((const void *)gemm_tile_kernel<S, EPI>,
+    (void)hipFuncSetAttribute((const void *)gemm_tile_kernel<S, EPI, TAIL>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS);
     attr = true;
   }
@@ -1203,10 +1204,20 @@ void launch_tile(const GemmPlan &p, const void *w, const void *si, const void *s
   // each XCD's L2 reads the larger operand once (0.5B o over 4096 tokens 16.3
   // -> 14.9 us, qkv 24.2 -> 22.6 us).
   const int rfast = (size_t)n * 2 * 16 > (size_t)rows * 9;
-  gemm_tile_kernel<S, EPI><<<p.grid, S::THREADS, S::LDS, WST_STREAM>>>(
+  gemm_tile_kernel<S, EPI, TAIL><<<p.grid, S::THREADS, S::LDS, WST_STREAM>>>(
       w, (const uint8_t *)si, (const uint32_t *)sb, (const uint16_t *)x, (const uint16_t *)bias,
       (float *)y, ws, in_f, out_f, n, accum, (n + S::BN - 1) / S::BN, (int)p.grid.x, p.gps, rfast,
       re);
+}
+
+template <class S, int EPI>
+void launch_tile(const GemmPlan &p, const void *w, const void *si, const void *sb, const void *x,
+                 const void *bias, void *y, float *ws, int in_f, int out_f, int rows, int n,
+                 int accum, const GtRope &re) {
+  if (in_f % GT_KC)
+    launch_tile_t<S, EPI, true>(p, w, si, sb, x, bias, y, ws, in_f, out_f, rows, n, accum, re);
+  else
+    launch_tile_t<S, EPI, false>(p, w, si, sb, x, bias, y, ws, in_f, out_f, rows, n, accum, re);
 }
 
 template <bool HIER, bool SWI>

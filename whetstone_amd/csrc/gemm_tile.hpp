@@ -1,5 +1,6 @@
 // Chunk GEMM tiles that dequantise int4-hier weights in registers:
-// y[j] (+)= W x[j] + b over rows of whole 128-column steps (in_f % 128 == 0).
+// y[j] (+)= W x[j] + b over rows of 128-column steps, the last whole or half
+// (in_f % 64 == 0, at least 128).
 // reference: chunk_gemm.cu:65-176.
 //
 // * A lane's MFMA operand (v_mfma_f32_32x32x16_f16: row lane % 32, eight
@@ -37,6 +38,8 @@ typedef _Float16 gt_h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 gt_h2 __attribute__((ext_vector_type(2)));
 typedef float gt_f16v __attribute__((ext_vector_type(16)));
 typedef uint32_t gt_u4 __attribute__((ext_vector_type(4)));
+
+typedef uint32_t gt_u32a2 __attribute__((aligned(2)));
 
 #define GT_KC 128           // columns per step: four int4-hier groups
 // VALU ops scheduled after each MFMA: a k-step's dequantisations over its MFMAs
@@ -96,7 +99,9 @@ struct GtW {
 // writes ws[y] when ws is given. nb token tiles, `tiles` tiles; rfast: row
 // tiles vary fastest. 32-bit offsets: n in_f 2, rows in_f / 2 and n out_f 4
 // are below 2^31 (the host checks).
-template <class S, int EPI>
+// TAIL: rows end in half a step (in_f % 128 == 64): the last step has groups 0
+// and 1 only; its groups 2 and 3 are weights of zero.
+template <class S, int EPI, bool TAIL>
 __global__ __launch_bounds__(S::THREADS, S::MT * S::NT > 8 ? 1 : 2) void gemm_tile_kernel(
     const void *__restrict__ qw, const uint8_t *__restrict__ si, const uint32_t *__restrict__ sb,
     const uint16_t *__restrict__ x, const uint16_t *__restrict__ bias, float *__restrict__ y,
@@ -121,7 +126,8 @@ __global__ __launch_bounds__(S::THREADS, S::MT * S::NT > 8 ? 1 : 2) void gemm_ti
   const int tm = rfast ? b % mb : b / nb, tn = rfast ? b / mb : b % nb;
   const int t0 = tn * S::BN;
   const int G = in_f >> 5;
-  const int step0 = blockIdx.y * sps, step1 = min(in_f / GT_KC, step0 + sps);
+  const int whole = in_f / GT_KC;  // whole steps of a row
+  const int step0 = blockIdx.y * sps, step1 = min(whole + (TAIL ? 1 : 0), step0 + sps);
 
   uint32_t woff[MT], ioff[MT];
   float ds[MT], dm[MT];
@@ -152,23 +158,37 @@ __global__ __launch_bounds__(S::THREADS, S::MT * S::NT > 8 ? 1 : 2) void gemm_ti
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)gt_lds;
 
+  // A tail step's second half re-reads its first (nothing past a row is read).
   auto load_x = [&](int st, int buf) {
     const uint16_t *xs = x + (size_t)st * GT_KC;
+    const bool tail = TAIL && st == whole;
     const uint32_t dst = lds0 + (uint32_t)buf * S::XBUF + (uint32_t)wave * (S::XDMA * 1024u);
 #pragma unroll
-    for (int i = 0; i < S::XDMA; ++i)
+    for (int i = 0; i < S::XDMA; ++i) {
+      uint32_t off = xoff[i];
+      if constexpr (TAIL) {
+        const int tl = (wave * S::XDMA + i) * 4 + (lane >> 4);
+        off -= tail ? (uint32_t)((lane ^ tl) & 8) * 16u : 0u;  // chunk 8 and on: chunk - 8
+      }
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                   ::"s"(dst + i * 1024u), "v"(xoff[i]), "s"(xs)
+                   ::"s"(dst + i * 1024u), "v"(off), "s"(xs)
                    : "memory");
+    }
   };
   auto load_w = [&](int st, GtW<MT> &w) {
     const char *qs = (const char *)qw + (size_t)st * (GT_KC / 2);
-    const uint8_t *is = si + (size_t)st * 4;
+    const bool tail = TAIL && st == whole;
+    // index bytes: a tail's two are the upper half of the word that ends with
+    // the row (rows of an odd number of group pairs are 2-byte aligned)
+    const uint8_t *is = si + (size_t)st * 4 - (tail ? 2 : 0);
 #pragma unroll
     for (int f = 0; f < MT; ++f) {
       w.q[f][0] = *(const gt_u4 *)(qs + woff[f]);
-      w.q[f][1] = *(const gt_u4 *)(qs + woff[f] + 32u);
-      w.ix[f] = *(const uint32_t *)(is + ioff[f]);
+      w.q[f][1] = *(const gt_u4 *)(qs + woff[f] + (tail ? 0u : 32u));
+      if constexpr (TAIL)
+        w.ix[f] = *(const gt_u32a2 *)(is + ioff[f]);
+      else
+        w.ix[f] = *(const uint32_t *)(is + ioff[f]);
     }
   };
   gt_f16v acc[MT][NT];
@@ -185,14 +205,17 @@ __global__ __launch_bounds__(S::THREADS, S::MT * S::NT > 8 ? 1 : 2) void gemm_ti
   // The step's eight MFMA k-steps i (groups 2 (i / 4) + half, word i % 4):
   // the next k-step's operands are read and dequantised under this one's
   // MFMAs.
-  auto compute = [&](const GtW<MT> &w, int buf) {
+  // A tail step's index bytes sit in the upper half of the word, and its groups
+  // 2 and 3 read scales of zero above it.
+  auto compute = [&](const GtW<MT> &w, int buf, int st) {
+    const int sh = 8 * half + (TAIL && st == whole ? 16 : 0);
     const unsigned char *xb = gt_lds + buf * S::XBUF + xbase;
     gt_h8 xf[2][NT], wf[2][MT];
     float sc[MT], sc16[MT], mm[MT];
     auto scales = [&](int s) {
 #pragma unroll
       for (int f = 0; f < MT; ++f) {
-        const uint32_t ix = (w.ix[f] >> (8 * half)) >> (16 * s);
+        const uint32_t ix = (w.ix[f] >> sh) >> (16 * s);
         sc[f] = ds[f] * (float)(ix & 0xFu);
         sc16[f] = sc[f] * 0.0625f;
         mm[f] = dm[f] * (float)((ix >> 4) & 0xFu);
@@ -255,16 +278,16 @@ __global__ __launch_bounds__(S::THREADS, S::MT * S::NT > 8 ? 1 : 2) void gemm_ti
     load_x(st + 1, 1);
     load_w(st + 1, w1);
     __builtin_amdgcn_sched_barrier(0);
-    compute(w0, 0);
+    compute(w0, 0, st);
     arrive(w1);
     load_x(min(st + 2, last), 0);
     load_w(min(st + 2, last), w0);
     __builtin_amdgcn_sched_barrier(0);
-    compute(w1, 1);
+    compute(w1, 1, st + 1);
   }
   if (st < step1) {
     arrive(w0);
-    compute(w0, 0);
+    compute(w0, 0, st);
   }
   // the clamped look-ahead DMA lands in LDS nobody reads any more; it must
   // land before the block ends and its LDS is given away
