@@ -134,3 +134,28 @@ def test_gemm_rope_epilogue_equals_gemm_then_rope_cache(orc, wk, in_f, n_q, n_kv
         out.append([t.numpy() for t in (qkv, k, v)])
     for a, e in zip(*out):
         assert np.array_equal(a.view(np.uint8), e.view(np.uint8))
+
+
+@pytest.mark.parametrize("in_f,out_f,n,accum", [(128, 1, 1, False), (192, 130, 33, True),
+                                                (896, 257, 65, False), (960, 1000, 256, True),
+                                                (4864, 96, 7, True), (256, 9000, 600, False)])
+def test_gemm_fp16_step_rows(orc, wk, in_f, out_f, n, accum):
+    """f16 weights over the same edges: the operands are exact, so only the f32
+    sums differ from float64 (at most in_f + 16 additions of relative 2^-24)."""
+    print(f"f16 gemm {in_f} -> {out_f}, {n} tokens", flush=True)
+    wb = f16(orc, orc.fixture_normal(65, 1, in_f * out_f, 0.05))
+    xb = f16(orc, orc.fixture_normal(65, 2, n * in_f, 1.0))
+    bb = f16(orc, orc.fixture_normal(65, 3, out_f, 0.3))
+    y0 = orc.fixture_normal(65, 4, (n + 1) * out_f, 1.0)
+    y = wk.DeviceBuffer.from_array(y0.copy())
+    wd, xd, bd = dev_f16(wk, wb), dev_f16(wk, xb), dev_f16(wk, bb)
+    ffi.call("wst_gemm_fp16", wd.ptr, xd.ptr, bd.ptr, y.ptr, in_f, out_f, n, int(accum))
+    w = wb.view(np.float16).astype(np.float64).reshape(out_f, in_f)
+    x = xb.view(np.float16).astype(np.float64).reshape(n, in_f)
+    ref = x @ w.T + bb.view(np.float16).astype(np.float64)
+    if accum:
+        ref = ref + y0.reshape(n + 1, out_f)[:n]
+    got = y.numpy().astype(np.float64).reshape(n + 1, out_f)
+    bound = (in_f + 16) * 2.0 ** -24 * (np.abs(x) @ np.abs(w).T + np.abs(ref) + 1)
+    assert float(np.max(np.abs(got[:n] - ref) / bound)) <= 1.0
+    assert np.array_equal(got[n], y0.reshape(n + 1, out_f)[n])

@@ -1052,13 +1052,14 @@ static int gemm_bn_override() {
   return v;
 }
 
-// The register-dequantising tiles take int4-hier rows of 128 columns or more in
-// whole 64-column halves of a step, with 4-byte aligned index bytes, within
-// their 32-bit offsets.
-bool tile_ok(const void *si, int in_f, int out_f, int rows, int n) {
+// The register tiles take rows of 128 columns or more in whole 64-column halves
+// of a step, int4-hier with 4-byte aligned index bytes, within their 32-bit
+// offsets.
+bool tile_ok(bool hier, const void *si, int in_f, int out_f, int rows, int n) {
   const size_t lim = (size_t)1 << 31;
-  return gemm_tiles_mode() == 1 && in_f % 64 == 0 && in_f >= GT_KC && !((uintptr_t)si & 3u) &&
-         (size_t)n * in_f * 2 < lim && (size_t)rows * (in_f / 2) < lim &&
+  return gemm_tiles_mode() == 1 && in_f % 64 == 0 && in_f >= GT_KC &&
+         (!hier || !((uintptr_t)si & 3u)) && (size_t)n * in_f * 2 < lim &&
+         (size_t)rows * (hier ? in_f / 2 : in_f * 2) < lim &&
          (size_t)n * out_f * 4 < lim && out_f <= (1 << 20);
 }
 
@@ -1069,13 +1070,16 @@ struct TileCost {
   int bm, bn;
   float lat, thr, fixed;
 };
-constexpr TileCost TILE_COST[2][3] = {
+constexpr TileCost TILE_COST[3][3] = {  // int4, int4 SwiGLU (and RoPE), f16
     {{GtBig::BM, GtBig::BN, 1.8f, 1.9f, 8.0f},
      {GtMid::BM, GtMid::BN, 0.7f, 0.75f, 4.5f},
      {GtLow::BM, GtLow::BN, 0.8f, 0.55f, 4.0f}},
     {{GtBig::BM, GtBig::BN, 1.8f, 1.9f, 6.0f},
      {GtMidSwi::BM, GtMidSwi::BN, 1.27f, 1.2f, 4.5f},
-     {GtLowSwi::BM, GtLowSwi::BN, 1.05f, 0.95f, 4.5f}}};
+     {GtLowSwi::BM, GtLowSwi::BN, 1.05f, 0.95f, 4.5f}},
+    {{GtBig::BM, GtBig::BN, 1e9f, 1e9f, 0.0f},  // (not built: its weights would not fit)
+     {GtMid::BM, GtMid::BN, 0.9f, 0.75f, 4.5f},
+     {GtLow::BM, GtLow::BN, 0.9f, 0.65f, 4.0f}}};
 
 // The tile and K split of the least estimated time: steps a block x what a
 // step takes with the blocks the fullest CU holds, the tile's fixed part, and
@@ -1087,13 +1091,16 @@ constexpr TileCost TILE_COST[2][3] = {
 // 20.9 / 18.7 / -; 7B gate|up x 232 101 / 101 / 130, x 30 53 / 38 / 33;
 // 896 -> 151936 x 30 49 / 28 / 22; 3584 -> 4608 x 30 unsplit low 29, split 7
 // ways 9 with its reduce.
-void plan_tile(GemmPlan &p, int in_f, int out_f, int rows, int pn, int n, bool swi,
+// form: the row of TILE_COST.
+enum { FORM_INT4 = 0, FORM_SWIGLU = 1, FORM_F16 = 2 };
+void plan_tile(GemmPlan &p, int in_f, int out_f, int rows, int pn, int n, int form,
                size_t max_part) {
+  const bool swi = form == FORM_SWIGLU;
   const int steps = (in_f + GT_KC - 1) / GT_KC, cus = wst_cu_count();
   float best = 0.0f;
   p.tile = TILE_OLD;
   for (int t = TILE_BIG; t <= TILE_LOW; ++t) {
-    const TileCost &c = TILE_COST[swi][t - 1];
+    const TileCost &c = TILE_COST[form][t - 1];
     const int tiles = ((rows + c.bm - 1) / c.bm) * ((pn + c.bn - 1) / c.bn);
     for (int want = 1; want <= (swi ? 1 : GM_MAXSPLIT) && want <= steps; ++want) {
       const int sps = (steps + want - 1) / want, splits = (steps + sps - 1) / sps;
@@ -1136,8 +1143,16 @@ GemmPlan plan_gemm(int in_f, int out_f, int n, bool hier = true, int rows = 0, b
   GemmPlan p;
   if (rows <= 0) rows = out_f;
   const int pn = plan_n > 0 && plan_n < n ? plan_n : n;
-  if (hier && tile_ok(si, in_f, out_f, rows, n)) {
-    plan_tile(p, in_f, out_f, rows, pn, n, swi, max_part);
+  // f16 weights for few tokens: the 64 x 64 tiles' loads, whole rows apart, are
+  // not slower there, and their K split finer (start -> tiles, us: 4864 -> 896
+  // x 16 tokens 8.8 -> 10.0, 3904 -> 13620 x 4 20.1 -> 22.7; but 18944 -> 3584
+  // x 16 39 -> 33, 896 -> 151936 x 16 56 -> 46, 4864 -> 896 x 256 19.3 -> 14.4).
+  const size_t wbytes = (size_t)rows * in_f * 2;
+  const bool f16_pays = pn > 64 || wbytes >= ((size_t)128 << 20) ||
+                        (pn > 32 && in_f >= 3072 && wbytes >= ((size_t)24 << 20));
+  if ((hier || f16_pays) && tile_ok(hier, si, in_f, out_f, rows, n)) {
+    plan_tile(p, in_f, out_f, rows, pn, n, !hier ? FORM_F16 : swi ? FORM_SWIGLU : FORM_INT4,
+              max_part);
     p.wide = false;
     p.nwv = 0;
     p.kg = 0;
@@ -1189,13 +1204,13 @@ GemmPlan plan_gemm(int in_f, int out_f, int n, bool hier = true, int rows = 0, b
   return p;
 }
 
-template <class S, int EPI, bool TAIL>
+template <class S, int EPI, bool TAIL, bool F16>
 void launch_tile_t(const GemmPlan &p, const void *w, const void *si, const void *sb, const void *x,
                  const void *bias, void *y, float *ws, int in_f, int out_f, int rows, int n,
                  int accum, const GtRope &re) {
   static bool attr = false;
   if (!attr) {
-    (void)hipFuncSetAttribute((const void *)gemm_tile_kernel<S, EPI, TAIL>,
+    (void)hipFuncSetAttribute((const void *)gemm_tile_kernel<S, EPI, TAIL, F16>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS);
     attr = true;
   }
@@ -1203,21 +1218,21 @@ void launch_tile_t(const GemmPlan &p, const void *w, const void *si, const void 
   // tiles an XCD, every row) where x outweighs the packed weights, so that
   // each XCD's L2 reads the larger operand once (0.5B o over 4096 tokens 16.3
   // -> 14.9 us, qkv 24.2 -> 22.6 us).
-  const int rfast = (size_t)n * 2 * 16 > (size_t)rows * 9;
-  gemm_tile_kernel<S, EPI, TAIL><<<p.grid, S::THREADS, S::LDS, WST_STREAM>>>(
+  const int rfast = (size_t)n * 2 * 16 > (size_t)rows * (F16 ? 32 : 9);
+  gemm_tile_kernel<S, EPI, TAIL, F16><<<p.grid, S::THREADS, S::LDS, WST_STREAM>>>(
       w, (const uint8_t *)si, (const uint32_t *)sb, (const uint16_t *)x, (const uint16_t *)bias,
       (float *)y, ws, in_f, out_f, n, accum, (n + S::BN - 1) / S::BN, (int)p.grid.x, p.gps, rfast,
       re);
 }
 
-template <class S, int EPI>
+template <class S, int EPI, bool F16 = false>
 void launch_tile(const GemmPlan &p, const void *w, const void *si, const void *sb, const void *x,
                  const void *bias, void *y, float *ws, int in_f, int out_f, int rows, int n,
                  int accum, const GtRope &re) {
   if (in_f % GT_KC)
-    launch_tile_t<S, EPI, true>(p, w, si, sb, x, bias, y, ws, in_f, out_f, rows, n, accum, re);
+    launch_tile_t<S, EPI, true, F16>(p, w, si, sb, x, bias, y, ws, in_f, out_f, rows, n, accum, re);
   else
-    launch_tile_t<S, EPI, false>(p, w, si, sb, x, bias, y, ws, in_f, out_f, rows, n, accum, re);
+    launch_tile_t<S, EPI, false, F16>(p, w, si, sb, x, bias, y, ws, in_f, out_f, rows, n, accum, re);
 }
 
 template <bool HIER, bool SWI>
@@ -1235,6 +1250,18 @@ void launch_gemm(const GemmPlan &p, const void *w, const void *si, const void *s
       if (p.tile == TILE_BIG) go(GtBig{});
       else if (p.tile == TILE_MID) go(Mid{});
       else go(Low{});
+      return;
+    }
+  }
+  if constexpr (!HIER) {
+    if (p.tile == TILE_MID) {
+      launch_tile<GtMid, GT_PLAIN, true>(p, w, si, sb, x, bias, y, ws, in_f, out_f, out_f, n, accum,
+                                         GtRope{});
+      return;
+    }
+    if (p.tile == TILE_LOW) {
+      launch_tile<GtLow, GT_PLAIN, true>(p, w, si, sb, x, bias, y, ws, in_f, out_f, out_f, n, accum,
+                                         GtRope{});
       return;
     }
   }
@@ -1442,7 +1469,7 @@ extern "C" wst_status_t wst_gemm_hier_rope_chunks(const void *qw, const void *si
     if (p.tile != TILE_OLD && p.splits == 1 && rope_epilogue_on() &&
         (head_dim == 64 || (head_dim == 128 && !q_norm_w && !k_norm_w)) &&
         (size_t)max_seq * head_dim * 2 < ((size_t)1 << 31)) {
-      plan_tile(p, in_f, out_f, out_f, n, n, true, 0);
+      plan_tile(p, in_f, out_f, out_f, n, n, FORM_SWIGLU, 0);
       p.grid = dim3((unsigned)(((out_f + p.bm - 1) / p.bm) * ((n + p.bn - 1) / p.bn)), 1, 1);
       const GtRope re{(uint16_t *)k_cache, (uint16_t *)v_cache, (const float *)cos_tab,
                       (const float *)sin_tab, (const uint16_t *)q_norm_w,

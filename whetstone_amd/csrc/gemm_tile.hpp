@@ -24,6 +24,10 @@
 //   weight row, so a store instruction writes whole 128-byte row pieces and
 //   needs no pass through LDS; a gate row and its up row (and a RoPE pair) sit
 //   in one lane.
+// * F16 weights (wst_gemm_fp16) run the same loop with the operand loaded as it
+//   is: 896 -> 151936 x 256 tokens 292 -> 173 us (each load instruction touches
+//   32 rows, which bounds it: the f16 products stay far from the matrix cores'
+//   rate).
 // * Every shape sums k in the same order, so a token's bits do not depend on
 //   the tile, only on the K split.
 //
@@ -43,7 +47,7 @@ typedef uint32_t gt_u32a2 __attribute__((aligned(2)));
 
 #define GT_KC 128           // columns per step: four int4-hier groups
 // VALU ops scheduled after each MFMA: a k-step's dequantisations over its MFMAs
-#define GT_VPM ((13 * MT + MT * NT - 1) / (MT * NT) + 1)
+#define GT_VPM (F16 ? 1 : (13 * MT + MT * NT - 1) / (MT * NT) + 1)
 #define GT_XROW (GT_KC * 2) // bytes of a token's step in LDS
 
 struct GtRope {
@@ -88,10 +92,11 @@ __device__ __forceinline__ gt_h8 gt_dequant(uint32_t w, float s, float s16, floa
   return r;
 }
 
-template <int MT>
+template <int MT, bool F16>
 struct GtW {
-  gt_u4 q[MT][2];   // groups half and 2 + half of the step
-  uint32_t ix[MT];  // the step's four index bytes
+  // int4: groups half and 2 + half of the step; f16: the eight k-steps' operands
+  gt_u4 q[MT][F16 ? 8 : 2];
+  uint32_t ix[MT];  // int4: the step's four index bytes
 };
 
 // qw/si/sb: the weights [rows][in_f] (rows = out_f, or 2 out_f for the SwiGLU
@@ -101,7 +106,10 @@ struct GtW {
 // are below 2^31 (the host checks).
 // TAIL: rows end in half a step (in_f % 128 == 64): the last step has groups 0
 // and 1 only; its groups 2 and 3 are weights of zero.
-template <class S, int EPI, bool TAIL>
+// F16: w is f16 [rows][in_f] (si and sb unused): a lane's operand is 16 bytes of
+// a row, loaded straight into registers; k-step i covers columns 16 i .. 16 i +
+// 15.
+template <class S, int EPI, bool TAIL, bool F16>
 __global__ __launch_bounds__(S::THREADS, S::MT * S::NT > 8 ? 1 : 2) void gemm_tile_kernel(
     const void *__restrict__ qw, const uint8_t *__restrict__ si, const uint32_t *__restrict__ sb,
     const uint16_t *__restrict__ x, const uint16_t *__restrict__ bias, float *__restrict__ y,
@@ -143,11 +151,17 @@ __global__ __launch_bounds__(S::THREADS, S::MT * S::NT > 8 ? 1 : 2) void gemm_ti
     } else {
       r = min(tm * S::BM + (wm * MT + f) * 32 + l32, out_f - 1);
     }
-    const uint32_t p = sb[r];
-    ds[f] = h2f((uint16_t)(p & 0xFFFFu)) * 16777216.0f;
-    dm[f] = -h2f((uint16_t)(p >> 16));
-    woff[f] = (uint32_t)r * (uint32_t)(in_f / 2) + (uint32_t)half * 16u;
-    ioff[f] = (uint32_t)r * (uint32_t)G;
+    if constexpr (F16) {
+      ds[f] = dm[f] = 0.0f;
+      woff[f] = (uint32_t)r * (uint32_t)(in_f * 2) + (uint32_t)half * 16u;
+      ioff[f] = 0;
+    } else {
+      const uint32_t p = sb[r];
+      ds[f] = h2f((uint16_t)(p & 0xFFFFu)) * 16777216.0f;
+      dm[f] = -h2f((uint16_t)(p >> 16));
+      woff[f] = (uint32_t)r * (uint32_t)(in_f / 2) + (uint32_t)half * 16u;
+      ioff[f] = (uint32_t)r * (uint32_t)G;
+    }
   }
   uint32_t xoff[S::XDMA];
 #pragma unroll
@@ -175,9 +189,18 @@ __global__ __launch_bounds__(S::THREADS, S::MT * S::NT > 8 ? 1 : 2) void gemm_ti
                    : "memory");
     }
   };
-  auto load_w = [&](int st, GtW<MT> &w) {
-    const char *qs = (const char *)qw + (size_t)st * (GT_KC / 2);
+  auto load_w = [&](int st, GtW<MT, F16> &w) {
     const bool tail = TAIL && st == whole;
+    if constexpr (F16) {
+      const char *ws_ = (const char *)qw + (size_t)st * (GT_KC * 2);
+#pragma unroll
+      for (int f = 0; f < MT; ++f)
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          w.q[f][i] = *(const gt_u4 *)(ws_ + woff[f] + (tail && i >= 4 ? i - 4 : i) * 32u);
+      return;
+    }
+    const char *qs = (const char *)qw + (size_t)st * (GT_KC / 2);
     // index bytes: a tail's two are the upper half of the word that ends with
     // the row (rows of an odd number of group pairs are 2-byte aligned)
     const uint8_t *is = si + (size_t)st * 4 - (tail ? 2 : 0);
@@ -201,18 +224,19 @@ __global__ __launch_bounds__(S::THREADS, S::MT * S::NT > 8 ? 1 : 2) void gemm_ti
 
   // token wn * NT * 32 + 32 t + l32, chunk c at slot c ^ (token % 16)
   const uint32_t xbase = (uint32_t)((wn * NT * 32 + l32) * GT_XROW);
-  const uint32_t xsw = (uint32_t)((4 * half) ^ (l32 & 15)) << 4;
+  const uint32_t xsw = (uint32_t)((F16 ? half : 4 * half) ^ (l32 & 15)) << 4;
   // The step's eight MFMA k-steps i (groups 2 (i / 4) + half, word i % 4):
   // the next k-step's operands are read and dequantised under this one's
   // MFMAs.
   // A tail step's index bytes sit in the upper half of the word, and its groups
   // 2 and 3 read scales of zero above it.
-  auto compute = [&](const GtW<MT> &w, int buf, int st) {
+  auto compute = [&](const GtW<MT, F16> &w, int buf, int st) {
     const int sh = 8 * half + (TAIL && st == whole ? 16 : 0);
     const unsigned char *xb = gt_lds + buf * S::XBUF + xbase;
     gt_h8 xf[2][NT], wf[2][MT];
     float sc[MT], sc16[MT], mm[MT];
     auto scales = [&](int s) {
+      if constexpr (F16) return;
 #pragma unroll
       for (int f = 0; f < MT; ++f) {
         const uint32_t ix = (w.ix[f] >> sh) >> (16 * s);
@@ -225,11 +249,19 @@ __global__ __launch_bounds__(S::THREADS, S::MT * S::NT > 8 ? 1 : 2) void gemm_ti
 #pragma unroll
       for (int t = 0; t < NT; ++t)
         xf[i & 1][t] = *(const gt_h8 *)(xb + t * 32 * GT_XROW +
-                                        (xsw ^ (uint32_t)((8 * (i >> 2) + (i & 3)) * 16)));
+                                        (xsw ^ (uint32_t)((F16 ? 2 * i : 8 * (i >> 2) + (i & 3)) * 16)));
     };
     auto make_w = [&](int i) {
 #pragma unroll
-      for (int f = 0; f < MT; ++f) wf[i & 1][f] = gt_dequant(w.q[f][i >> 2][i & 3], sc[f], sc16[f], mm[f]);
+      for (int f = 0; f < MT; ++f) {
+        if constexpr (F16) {
+          // (a tail step's second half: weights of zero)
+          const uint32_t keep = TAIL && st == whole && i >= 4 ? 0u : ~0u;
+          wf[i & 1][f] = __builtin_bit_cast(gt_h8, TAIL ? w.q[f][i] & (gt_u4)keep : w.q[f][i]);
+        } else {
+          wf[i & 1][f] = gt_dequant(w.q[f][i >> 2][i & 3], sc[f], sc16[f], mm[f]);
+        }
+      }
     };
     scales(0);
     read_x(0);
@@ -258,17 +290,25 @@ __global__ __launch_bounds__(S::THREADS, S::MT * S::NT > 8 ? 1 : 2) void gemm_ti
       }
     }
   };
-  auto arrive = [&](GtW<MT> &w) {
+  auto arrive = [&](GtW<MT, F16> &w) {
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int f = 0; f < MT; ++f)
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)"
-                   : "+v"(w.q[f][0]), "+v"(w.q[f][1]), "+v"(w.ix[f])::"memory");
+    for (int f = 0; f < MT; ++f) {
+      if constexpr (F16) {
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)"
+                     : "+v"(w.q[f][0]), "+v"(w.q[f][1]), "+v"(w.q[f][2]), "+v"(w.q[f][3]),
+                       "+v"(w.q[f][4]), "+v"(w.q[f][5]), "+v"(w.q[f][6]), "+v"(w.q[f][7])
+                     ::"memory");
+      } else {
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)"
+                     : "+v"(w.q[f][0]), "+v"(w.q[f][1]), "+v"(w.ix[f])::"memory");
+      }
+    }
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
 
-  GtW<MT> w0, w1;
+  GtW<MT, F16> w0, w1;
   load_x(step0, 0);
   load_w(step0, w0);
   const int last = step1 - 1;
