@@ -38,7 +38,6 @@
 #include "gemm_tile.hpp"
 
 #include <mutex>
-#include <type_traits>
 
 #define HGROUP 32
 #define GM_BM 64
@@ -1014,14 +1013,15 @@ void set_lds_attr() {
 
 // Register-dequantising tiles (gemm_tile.hpp), four waves each: 256 rows x 128
 // tokens (waves of 64 x 128), 128 rows x 64 tokens (32 x 64) and 128 rows x 32
-// tokens (32 x 32); the SwiGLU forms pair a gate and an up fragment in every
-// wave, so their small tiles are 256 weight rows too.
+// tokens (32 x 32). SwiGLU also takes 256 weight rows x 64 tokens (64 x 64,
+// TILE_PAIR); the RoPE epilogue wants a rotation pair in every wave, so its
+// small tiles are all 256 rows.
 using GtBig = GtShape<4, 1, 2, 4>;
 using GtMid = GtShape<4, 1, 1, 2>;
 using GtLow = GtShape<4, 1, 1, 1>;
-using GtMidSwi = GtShape<4, 1, 2, 2>;
-using GtLowSwi = GtShape<4, 1, 2, 1>;
-enum GemmTile { TILE_OLD = 0, TILE_BIG = 1, TILE_MID = 2, TILE_LOW = 3 };
+using GtMidPair = GtShape<4, 1, 2, 2>;
+using GtLowPair = GtShape<4, 1, 2, 1>;
+enum GemmTile { TILE_OLD = 0, TILE_BIG = 1, TILE_MID = 2, TILE_LOW = 3, TILE_PAIR = 4 };
 
 struct GemmPlan {
   int tile;  // GemmTile; TILE_OLD: the LDS tiles (wide or not, below)
@@ -1070,39 +1070,49 @@ struct TileCost {
   int bm, bn;
   float lat, thr, fixed;
 };
-constexpr TileCost TILE_COST[3][3] = {  // int4, int4 SwiGLU (and RoPE), f16
+constexpr TileCost NO_TILE = {256, 64, 1e9f, 1e9f, 0.0f};
+constexpr TileCost TILE_COST[4][4] = {  // int4, int4 SwiGLU, f16, RoPE epilogue
     {{GtBig::BM, GtBig::BN, 1.8f, 1.9f, 8.0f},
      {GtMid::BM, GtMid::BN, 0.7f, 0.75f, 4.5f},
-     {GtLow::BM, GtLow::BN, 0.8f, 0.55f, 4.0f}},
+     {GtLow::BM, GtLow::BN, 0.8f, 0.55f, 4.0f},
+     NO_TILE},
     {{GtBig::BM, GtBig::BN, 1.8f, 1.9f, 6.0f},
-     {GtMidSwi::BM, GtMidSwi::BN, 1.27f, 1.2f, 4.5f},
-     {GtLowSwi::BM, GtLowSwi::BN, 1.05f, 0.95f, 4.5f}},
-    {{GtBig::BM, GtBig::BN, 1e9f, 1e9f, 0.0f},  // (not built: its weights would not fit)
+     {GtMid::BM, GtMid::BN, 0.7f, 0.75f, 5.0f},
+     {GtLow::BM, GtLow::BN, 0.7f, 0.5f, 4.5f},
+     {GtMidPair::BM, GtMidPair::BN, 1.27f, 1.2f, 4.5f}},
+    {NO_TILE,  // (f16 weights of the big tile would not fit its registers)
      {GtMid::BM, GtMid::BN, 0.9f, 0.75f, 4.5f},
-     {GtLow::BM, GtLow::BN, 0.9f, 0.65f, 4.0f}}};
+     {GtLow::BM, GtLow::BN, 0.9f, 0.65f, 4.0f},
+     NO_TILE},
+    {{GtBig::BM, GtBig::BN, 1.8f, 1.9f, 6.0f},
+     {GtMidPair::BM, GtMidPair::BN, 1.27f, 1.2f, 4.5f},
+     {GtLowPair::BM, GtLowPair::BN, 1.05f, 0.95f, 4.5f},
+     NO_TILE}};
 
 // The tile and K split of the least estimated time: steps a block x what a
 // step takes with the blocks the fullest CU holds, the tile's fixed part, and
 // for a split a reduce launch and each further partial's way out and back (4
 // TB/s; the residual and qkv forms write one partial and reduce it anyway).
-// The partials stay below max_part bytes; the SwiGLU form never splits. A
+// The partials stay below max_part bytes; the SwiGLU and RoPE epilogues never
+// split. A
 // token's bits depend on the split only, not on the tile.
 // Where it lies, measured in us (big / mid / low): 896 -> 1152 x 4096 tokens
-// 20.9 / 18.7 / -; 7B gate|up x 232 101 / 101 / 130, x 30 53 / 38 / 33;
+// 20.9 / 18.7 / -; 7B gate|up x 30 53 / 40 / 26; 0.5B gate|up x 256 18 / 13.9 /
+// -, pair 12.9;
 // 896 -> 151936 x 30 49 / 28 / 22; 3584 -> 4608 x 30 unsplit low 29, split 7
 // ways 9 with its reduce.
 // form: the row of TILE_COST.
-enum { FORM_INT4 = 0, FORM_SWIGLU = 1, FORM_F16 = 2 };
+enum { FORM_INT4 = 0, FORM_SWIGLU = 1, FORM_F16 = 2, FORM_ROPE = 3 };
 void plan_tile(GemmPlan &p, int in_f, int out_f, int rows, int pn, int n, int form,
                size_t max_part) {
-  const bool swi = form == FORM_SWIGLU;
+  const bool whole = form == FORM_SWIGLU || form == FORM_ROPE;
   const int steps = (in_f + GT_KC - 1) / GT_KC, cus = wst_cu_count();
   float best = 0.0f;
   p.tile = TILE_OLD;
-  for (int t = TILE_BIG; t <= TILE_LOW; ++t) {
+  for (int t = TILE_BIG; t <= TILE_PAIR; ++t) {
     const TileCost &c = TILE_COST[form][t - 1];
     const int tiles = ((rows + c.bm - 1) / c.bm) * ((pn + c.bn - 1) / c.bn);
-    for (int want = 1; want <= (swi ? 1 : GM_MAXSPLIT) && want <= steps; ++want) {
+    for (int want = 1; want <= (whole ? 1 : GM_MAXSPLIT) && want <= steps; ++want) {
       const int sps = (steps + want - 1) / want, splits = (steps + sps - 1) / sps;
       if (splits > 1 && (size_t)splits * n * out_f * 4 > max_part) break;
       if (gemm_split_cap() > 0 && splits > gemm_split_cap()) break;
@@ -1241,15 +1251,14 @@ void launch_gemm(const GemmPlan &p, const void *w, const void *si, const void *s
   if constexpr (HIER) {
     if (p.tile != TILE_OLD) {
       constexpr int E = SWI ? GT_SWIGLU : GT_PLAIN;
-      using Mid = std::conditional_t<SWI, GtMidSwi, GtMid>;
-      using Low = std::conditional_t<SWI, GtLowSwi, GtLow>;
       auto go = [&](auto shape) {
         launch_tile<decltype(shape), E>(p, w, si, sb, x, bias, y, ws, in_f, out_f,
                                         SWI ? 2 * out_f : out_f, n, accum, GtRope{});
       };
       if (p.tile == TILE_BIG) go(GtBig{});
-      else if (p.tile == TILE_MID) go(Mid{});
-      else go(Low{});
+      else if (p.tile == TILE_MID) go(GtMid{});
+      else if (p.tile == TILE_LOW) go(GtLow{});
+      else if constexpr (SWI) go(GtMidPair{});
       return;
     }
   }
@@ -1469,7 +1478,7 @@ extern "C" wst_status_t wst_gemm_hier_rope_chunks(const void *qw, const void *si
     if (p.tile != TILE_OLD && p.splits == 1 && rope_epilogue_on() &&
         (head_dim == 64 || (head_dim == 128 && !q_norm_w && !k_norm_w)) &&
         (size_t)max_seq * head_dim * 2 < ((size_t)1 << 31)) {
-      plan_tile(p, in_f, out_f, out_f, n, n, FORM_SWIGLU, 0);
+      plan_tile(p, in_f, out_f, out_f, n, n, FORM_ROPE, 0);
       p.grid = dim3((unsigned)(((out_f + p.bm - 1) / p.bm) * ((n + p.bn - 1) / p.bn)), 1, 1);
       const GtRope re{(uint16_t *)k_cache, (uint16_t *)v_cache, (const float *)cos_tab,
                       (const float *)sin_tab, (const uint16_t *)q_norm_w,
@@ -1483,8 +1492,8 @@ extern "C" wst_status_t wst_gemm_hier_rope_chunks(const void *qw, const void *si
                                                    out_f, out_f, n, 0, re);
       };
       if (p.tile == TILE_BIG) go(GtBig{});
-      else if (p.tile == TILE_MID) go(GtMidSwi{});
-      else go(GtLowSwi{});
+      else if (p.tile == TILE_MID) go(GtMidPair{});
+      else go(GtLowPair{});
       WST_TRY_KERNEL("wst_gemm_hier_rope_chunk");
       return WST_OK;
     }
