@@ -47,8 +47,9 @@ def test_gemm_odd_group_counts(orc, wk, in_f, out_f, n, accum):
     _check(y.numpy().astype(np.float64).reshape(n, out_f), x, w, ref)
 
 
-# rows of 128-column steps: one step, an odd and an even count of them; one row, a row tile's edge and one past it; one token, a token tile's edge
-# and one past it; K split (long rows) with and without the accumulate
+# rows of 128-column steps: one step, an odd and an even count of them; one
+# row, a row tile's edge and one past it; one token, a token tile's edge and one
+# past it; K split (long rows) with and without the accumulate
 @pytest.mark.parametrize("in_f,out_f,n,accum", [(128, 1, 1, False), (256, 256, 128, True),
                                                 (384, 257, 129, False), (896, 127, 127, True),
                                                 (1152, 130, 70, False), (4864, 896, 256, True),
@@ -159,3 +160,35 @@ def test_gemm_fp16_step_rows(orc, wk, in_f, out_f, n, accum):
     bound = (in_f + 16) * 2.0 ** -24 * (np.abs(x) @ np.abs(w).T + np.abs(ref) + 1)
     assert float(np.max(np.abs(got[:n] - ref) / bound)) <= 1.0
     assert np.array_equal(got[n], y0.reshape(n + 1, out_f)[n])
+
+
+# rows that end in half a step: each column meets its own weight once, so an
+# infinite x gives the sign's infinity and leaves the other tokens alone
+@pytest.mark.parametrize("kind", ["hier", "fp16"])
+@pytest.mark.parametrize("in_f,out_f,n", [(192, 40, 70), (960, 257, 130)])
+def test_gemm_half_step_rows_infinite_x(orc, wk, kind, in_f, out_f, n):
+    print(f"{kind} gemm {in_f} -> {out_f}, {n} tokens, Inf in x", flush=True)
+    rng = np.random.default_rng(66)
+    x = rng.standard_normal((n, in_f)).astype(np.float16)
+    y = wk.DeviceBuffer(n * out_f, np.float32)
+    if kind == "hier":
+        p, _ = orc.quantize(orc.fixture_normal(66, 1, in_f * out_f), in_f, out_f)
+        lin = wk.QuantLinearHier.from_packed(p)
+        w = orc.dequantize(p).astype(np.float16).astype(np.float64).reshape(out_f, in_f)
+    else:
+        wb = f16(orc, orc.fixture_normal(66, 1, in_f * out_f, 0.05))
+        wd = dev_f16(wk, wb)
+        w = wb.view(np.float16).astype(np.float64).reshape(out_f, in_f)
+    tok, col = n // 2, in_f - 1 - n % 64
+    x[tok, col] = np.inf
+    xd = dev_f16(wk, x.view(np.uint16).reshape(-1))
+    if kind == "hier":
+        ffi.call("wst_gemm_int4_hier", lin.qw.ptr, lin.si.ptr, lin.sb.ptr, xd.ptr, None, y.ptr,
+                 in_f, out_f, n, 0)
+    else:
+        ffi.call("wst_gemm_fp16", wd.ptr, xd.ptr, None, y.ptr, in_f, out_f, n, 0)
+    got = y.numpy().reshape(n, out_f)
+    clear = np.abs(w[:, col]) > 1e-4  # (a weight that rounds to zero times Inf is NaN)
+    assert clear.sum() > out_f // 2
+    assert np.array_equal(got[tok][clear], np.sign(w[clear, col]).astype(np.float32) * np.inf)
+    assert np.all(np.isfinite(np.delete(got, tok, axis=0)))

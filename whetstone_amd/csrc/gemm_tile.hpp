@@ -252,9 +252,13 @@ __global__ __launch_bounds__(S::THREADS, S::MT * S::NT > 8 ? 1 : 2) void gemm_ti
     };
     auto read_x = [&](int i) {
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
-        xf[i & 1][t] = *(const gt_h8 *)(xb + t * 32 * GT_XROW +
-                                        (xsw ^ (uint32_t)((F16 ? 2 * i : 8 * (i >> 2) + (i & 3)) * 16)));
+      for (int t = 0; t < NT; ++t) {
+        gt_u4 v = *(const gt_u4 *)(xb + t * 32 * GT_XROW +
+                                   (xsw ^ (uint32_t)((F16 ? 2 * i : 8 * (i >> 2) + (i & 3)) * 16)));
+        // (a tail step's second half: x of zero too, as 0 * Inf is NaN)
+        if (TAIL && i >= 4) v &= (gt_u4)(st == whole ? 0u : ~0u);
+        xf[i & 1][t] = __builtin_bit_cast(gt_h8, v);
+      }
     };
     auto make_w = [&](int i) {
 #pragma unroll
