@@ -213,8 +213,9 @@ wst_status_t wst_gemm_hier_rope_chunks(const void *qw, const void *si, const voi
                                        const void *k_norm_w, float eps, int32_t plan_n);
 
 /* wst_attn_chunk over n tokens that hold several chunks, each token with the
- * bits a call of plan_n tokens gives it (the planned count picks how the keys
- * are split into partial sums); plan_n = 0 or n is wst_attn_chunk. */
+ * bits a call of plan_n tokens gives it whatever its position (the planned count
+ * picks how the keys are split into partial sums). plan_n = 0 is wst_attn_chunk:
+ * a call by itself, which also takes another kernel over few positions. */
 wst_status_t wst_attn_chunks(const void *qkv, const void *k_cache, const void *v_cache,
                              void *out, int32_t n_q, int32_t n_kv, int32_t head_dim,
                              int32_t pos0, int32_t n, int32_t max_seq, float scale,
@@ -235,9 +236,10 @@ wst_status_t wst_stream_read(const void *buf, size_t bytes, void *sink);
  * forbid hipMalloc): wst_gemm_int4_hier with the same arguments and the same
  * kernels, but its split-K partial sums go to a static 24 MiB device array
  * (one per GPU, held until the process ends) instead of the library's lazily
- * allocated scratch. Nothing is allocated or freed. A shape whose partials
- * need more than 24 MiB is refused with WST_ERR_SHAPE (the split plan keeps
- * them below (CUs + output tiles) x 64 KiB, under 24 MiB on 256 CUs). Every call on
+ * allocated scratch. Nothing is allocated or freed. The sum over K is split no
+ * further than the array holds (wst_gemm_int4_hier's own bound is 256 MiB, so
+ * the two may add a large output in another order); a shape whose partials need
+ * more all the same is refused with WST_ERR_SHAPE (none does on 256 CUs). Every call on
  * one GPU shares that array: calls that overlap on one GPU (other threads'
  * streams) race. The partials are fully written before they are read, so no
  * state carries over between calls. */

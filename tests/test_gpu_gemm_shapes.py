@@ -192,3 +192,57 @@ def test_gemm_half_step_rows_infinite_x(orc, wk, kind, in_f, out_f, n):
     assert clear.sum() > out_f // 2
     assert np.array_equal(got[tok][clear], np.sign(w[clear, col]).astype(np.float32) * np.inf)
     assert np.all(np.isfinite(np.delete(got, tok, axis=0)))
+
+
+@pytest.mark.parametrize("hd,n_q,n_kv,pos0,n", [(64, 14, 2, 1702, 37), (128, 28, 4, 900, 37),
+                                                (128, 28, 4, 5, 37)])
+def test_attn_chunk_output_between_words(orc, wk, hd, n_q, n_kv, pos0, n):
+    """An output that starts on an odd f16: the same values as an aligned one,
+    and nothing beside them."""
+    qkv = wk.DeviceBuffer.from_array(orc.fixture_normal(67, 1, n * (n_q + 2 * n_kv) * hd, 1.0))
+    k, v = (dev_f16(wk, f16(orc, orc.fixture_normal(67, i, n_kv * 1800 * hd, 1.0))) for i in (2, 3))
+    res = []
+    for shift in (0, 1):
+        out = wk.DeviceBuffer.from_array(np.full(n * n_q * hd + 2, 7.0, np.float16))
+        ffi.call("wst_attn_chunk", qkv.ptr, k.ptr, v.ptr, out.at(shift), n_q, n_kv, hd, pos0,
+                 n, 1800, hd ** -0.5)
+        o = out.numpy()
+        assert np.all(o[:shift] == 7.0) and np.all(o[n * n_q * hd + shift:] == 7.0)
+        res.append(o[shift:n * n_q * hd + shift].view(np.uint16))
+    assert np.array_equal(*res)
+
+
+@pytest.mark.parametrize("hd,n_q,n_kv,pos0,n", [(128, 28, 4, 645, 7), (128, 28, 4, 652, 7),
+                                                (128, 8, 8, 1001, 256), (128, 4, 2, 0, 131),
+                                                (128, 4, 4, 0, 1), (64, 14, 2, 300, 33),
+                                                (64, 8, 8, 1687, 6), (64, 8, 8, 1688, 6),
+                                                (64, 14, 2, 677, 511), (64, 14, 2, 0, 512)])
+def test_attn_chunk_positions(orc, wk, hd, n_q, n_kv, pos0, n):
+    """Both kernels on both sides of the rule that picks one, a wave's last tiles
+    empty or partly attended, NaN past the attended end, against float64.
+
+    Bound: P is rounded to f16 (2^-11 of each weight), the scores keep 22 bits
+    of |q||k| (scores of order 1: 2^-13 allowed), the output is rounded to f16."""
+    print(f"chunk attention hd {hd}, {n} tokens at {pos0}", flush=True)
+    max_seq, g = pos0 + n + 40, n_q // n_kv
+    rng = np.random.default_rng(68)
+    qkv = rng.standard_normal((n, n_q + 2 * n_kv, hd)).astype(np.float32)
+    k, v = (rng.standard_normal((n_kv, max_seq, hd)).astype(np.float16) for _ in range(2))
+    k[:, pos0 + n:] = np.nan
+    v[:, pos0 + n:] = np.nan
+    kd, vd = (dev_f16(wk, t.view(np.uint16).reshape(-1)) for t in (k, v))
+    qd = wk.DeviceBuffer.from_array(qkv.reshape(-1))
+    out = wk.DeviceBuffer(n * n_q * hd, np.float16)
+    ffi.call("wst_attn_chunk", qd.ptr, kd.ptr, vd.ptr, out.ptr, n_q, n_kv, hd, pos0, n, max_seq,
+             hd ** -0.5)
+    got = out.numpy().astype(np.float64).reshape(n, n_q, hd)
+    for h in range(n_q):
+        kh, vh = (t[h // g, :pos0 + n].astype(np.float64) for t in (k, v))
+        s = qkv[:, h].astype(np.float64) @ kh.T * hd ** -0.5
+        s[np.arange(pos0 + n)[None] > pos0 + np.arange(n)[:, None]] = -np.inf
+        p = np.exp(s - s.max(axis=1, keepdims=True))
+        p /= p.sum(axis=1, keepdims=True)
+        ref, mag = p @ vh, p @ np.abs(vh)
+        bound = (2.0 ** -11 + 2.0 ** -13) * mag + 2.0 ** -11 * np.abs(ref) + 2.0 ** -24
+        worst = float(np.max(np.abs(got[:, h] - ref) / bound))
+        assert worst <= 1.0, (h, worst)

@@ -175,8 +175,8 @@ __global__ __launch_bounds__(256) void attn_chunk_kernel(
 // 32 tokens of one head a block with K and V staged through registers (heads,
 // head_dim, tokens at position): 14/2 of 64, 4096 at 0: 79 -> 63; 14/2 of 64,
 // 256 at 3840: 21.8 -> 18.3; 28/4 of 128, 243 at 1792: 33 -> 21; 28/4 of 128,
-// 4096 at 0: 285 -> 245, 1000 at 0: 39 -> 33. A short prompt's one or two
-// tiles pay 0.8 us more for the merge (100 tokens at 0: 4.7 -> 5.5).
+// 4096 at 0: 285 -> 245, 1000 at 0: 39 -> 33. Over few positions the
+// launch's fixed parts count and the short kernel below is the faster one.
 typedef _Float16 ac_h8 __attribute__((ext_vector_type(8)));
 typedef short ac_s4 __attribute__((ext_vector_type(4)));
 typedef float ac_f16v __attribute__((ext_vector_type(16)));
@@ -399,35 +399,276 @@ __global__ __launch_bounds__((64 * RW * G), (HD == 64 ? 4 : 2)) void attn_chunk_
             make_float4(o[f][i], o[f][i + 1], o[f][i + 2], o[f][i + 3]);
   }
   __syncthreads();
-  // Two dims a thread, 4-byte stores.
+  // 2 G threads a row, four dims of every 8 G each. A row's weights, sum and
+  // quotients are one chain for all of a thread's dims (two dims a thread in
+  // 32 RW / 4 passes cost 0.4 us a pass: 28/4 heads of 128, 7 tokens at 0, 7.7
+  // us whole; 6.6 now). 8-byte stores, or 2-byte ones where out starts
+  // off 8 bytes.
+  const bool whole_words = ((uintptr_t)out & 7u) == 0;
   const int live = min(32 * RW, rows - rb);
-  constexpr int PER = S::THREADS / (HD / 2);  // rows a pass
-  const int d = 2 * (tid % (HD / 2));
+  constexpr int TPR = 2 * S::GROUPS, ND = HD / (4 * TPR);
+  static_assert(S::THREADS == TPR * 32 * RW && ND * 4 * TPR == HD, "every dim once");
+  const int r = tid / TPR, d0 = 4 * (tid % TPR);
+  const float *p = mb + r * S::MR;
+  float mw[S::GROUPS], M = -INFINITY, den = 0.0f;
+  float4 num[ND];
 #pragma unroll
-  for (int k = 0; k < 32 * RW / PER; ++k) {
-    const int r = tid / (HD / 2) + k * PER;
-    if (r >= live) continue;
-    const float *p = mb + r * S::MR;
-    float mw[S::GROUPS], M = -INFINITY;
+  for (int k = 0; k < ND; ++k) num[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll
-    for (int w = 0; w < S::GROUPS; ++w) {
-      mw[w] = p[w * 32 * RW * S::MR + HD];
-      M = fmaxf(M, mw[w]);
-    }
-    float n0 = 0.0f, n1 = 0.0f, den = 0.0f;
-#pragma unroll
-    for (int w = 0; w < S::GROUPS; ++w) {
-      const float *pw = p + w * 32 * RW * S::MR;
-      const float2 v = *(const float2 *)(pw + d);
-      const float f = mw[w] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mw[w] - M);  // base 2
-      n0 = fmaf(v.x, f, n0);
-      n1 = fmaf(v.y, f, n1);
-      den = fmaf(pw[HD + 1], f, den);
-    }
-    const int tk = (rb + r) / gqa, hd = kvh * gqa + (rb + r) % gqa;
-    *(uint32_t *)(out + ((size_t)tk * n_q + hd) * HD + d) =
-        (uint32_t)f2h(n0 / den) | ((uint32_t)f2h(n1 / den) << 16);
+  for (int w = 0; w < S::GROUPS; ++w) {
+    mw[w] = p[w * 32 * RW * S::MR + HD];
+    M = fmaxf(M, mw[w]);
   }
+#pragma unroll
+  for (int w = 0; w < S::GROUPS; ++w) {
+    const float *pw = p + w * 32 * RW * S::MR;
+    const float f = mw[w] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mw[w] - M);  // base 2
+    den = fmaf(pw[HD + 1], f, den);
+#pragma unroll
+    for (int k = 0; k < ND; ++k) {
+      const float4 v = *(const float4 *)(pw + d0 + 4 * TPR * k);
+      num[k].x = fmaf(v.x, f, num[k].x);
+      num[k].y = fmaf(v.y, f, num[k].y);
+      num[k].z = fmaf(v.z, f, num[k].z);
+      num[k].w = fmaf(v.w, f, num[k].w);
+    }
+  }
+  if (r >= live) return;
+  const int tk = (rb + r) / gqa, hd = kvh * gqa + (rb + r) % gqa;
+  uint16_t *op = out + ((size_t)tk * n_q + hd) * HD + d0;
+#pragma unroll
+  for (int k = 0; k < ND; ++k, op += 4 * TPR) {
+    const uint16_t h[4] = {f2h(num[k].x / den), f2h(num[k].y / den), f2h(num[k].z / den),
+                           f2h(num[k].w / den)};
+    if (whole_words)
+      *(uint2 *)op = make_uint2((uint32_t)h[0] | ((uint32_t)h[1] << 16),
+                                (uint32_t)h[2] | ((uint32_t)h[3] << 16));
+    else
+#pragma unroll
+      for (int i = 0; i < 4; ++i) op[i] = h[i];
+  }
+}
+
+// ------------------------------------- chunk attention over few positions
+//
+// The same attention for a chunk over a short cache: a block per (query head,
+// 16 tokens), four waves taking key tiles of 32 positions round-robin on
+// v_mfma_f32_16x16x32_f16, K and V staged through registers, merged once
+// through LDS. Its tile is a shorter chain than the kernel above (16 rows a wave
+// instead of 32: half the MFMA time) on several times the blocks, which is what
+// counts while a wave has a few tiles only. Scores, lazy maximum, P and the
+// transposing V reads are those above; keys past the attended end read zeros
+// through the buffer range check.
+typedef float as_f4 __attribute__((ext_vector_type(4)));
+typedef uint32_t as_u4 __attribute__((ext_vector_type(4)));
+
+#define AS_WAVES 4
+
+template <int HD>
+struct AsShape {
+  static constexpr int KS = HD / 32;              // k-steps of the scores
+  static constexpr int NT = HD / 16;              // 16-dim output tiles
+  static constexpr int VR = HD + 16;              // V row stride (halves)
+  static constexpr int KR = HD + 8;               // K row stride (halves)
+  static constexpr int VU = AC_KT * HD / 8 / 64;  // 16-byte K and V pieces per lane per tile
+  static constexpr int TILES = AC_KT * VR + AC_KT * KR;
+  static constexpr int MERGE = 16 * (HD + 2) * 2;  // the merge rows (floats), in halves
+  static constexpr int WAVE = TILES > MERGE ? TILES : MERGE;
+  static constexpr int LDS = AS_WAVES * WAVE * 2;
+};
+
+template <int HD, bool PLO>
+__global__ __launch_bounds__(AS_WAVES * 64) void attn_chunk_short_kernel(
+    const float *__restrict__ qkv, const uint16_t *__restrict__ k_cache,
+    const uint16_t *__restrict__ v_cache, uint16_t *__restrict__ out, int n_q, int n_kv,
+    int pos0, int n, int max_seq, float scale) {
+  using S = AsShape<HD>;
+  extern __shared__ __align__(16) unsigned char ac_lds[];
+  // Token groups in reverse order: the longest blocks start first.
+  const int head = blockIdx.x, t0 = (gridDim.y - 1 - blockIdx.y) * 16;
+  const int kvh = head / (n_q / n_kv);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: the tile loop is scalar
+  const int r16 = lane & 15, kg = lane >> 4;
+  uint16_t *vs = (uint16_t *)ac_lds + wave * S::WAVE;  // V tile [AC_KT][VR], row-major
+  uint16_t *ks = vs + AC_KT * S::VR;                   // K tile [AC_KT][KR], row-major
+  const int stride_row = (n_q + 2 * n_kv) * HD;
+  const uint16_t *kb = k_cache + (size_t)kvh * max_seq * HD;
+  const uint16_t *vb = v_cache + (size_t)kvh * max_seq * HD;
+
+  // q^T of token t0 + r16 as the B operand: dims 32s + 8kg + i, hi and lo
+  const float qscale = scale * 1.44269504088896340736f;
+  ac_h8 qh[S::KS], ql[S::KS];
+  {
+    const float *q = qkv + (size_t)min(t0 + r16, n - 1) * stride_row + (size_t)head * HD;
+#pragma unroll
+    for (int s = 0; s < S::KS; ++s) {
+      const float4 a = *(const float4 *)(q + 32 * s + 8 * kg);
+      const float4 b = *(const float4 *)(q + 32 * s + 8 * kg + 4);
+      const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float x = v[i] * qscale;
+        const _Float16 h = (_Float16)x;
+        qh[s][i] = h;
+        ql[s][i] = (_Float16)(x - (float)h);
+      }
+    }
+  }
+  const int kend = min(pos0 + min(t0 + 16, n), max_seq);  // positions [0, kend) are attended
+  const int ntiles = (kend + AC_KT - 1) / AC_KT;
+  const int lim = pos0 + t0 + r16;  // the last position this lane's token attends
+
+  // The whole byte offset goes in the vector offset, which is what the range
+  // check compares with the buffer's size.
+  const uint32_t kv_bytes = (uint32_t)kend * HD * 2u;
+  const __amdgpu_buffer_rsrc_t krs =
+      __builtin_amdgcn_make_buffer_rsrc((void *)kb, 0, (int)kv_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t vrs =
+      __builtin_amdgcn_make_buffer_rsrc((void *)vb, 0, (int)kv_bytes, 0x00020000);
+  const uint32_t voff = (uint32_t)lane * 16u;  // rows of a tile are contiguous
+  as_u4 kr[S::VU], vr[S::VU];
+  auto load_tile = [&](int kt) {
+    const uint32_t so = (uint32_t)kt * (AC_KT * HD * 2);
+#pragma unroll
+    for (int j = 0; j < S::VU; ++j)
+      kr[j] = __builtin_amdgcn_raw_buffer_load_b128(krs, so + voff + j * 1024, 0, 0);
+#pragma unroll
+    for (int j = 0; j < S::VU; ++j)
+      vr[j] = __builtin_amdgcn_raw_buffer_load_b128(vrs, so + voff + j * 1024, 0, 0);
+  };
+
+  float m = -INFINITY, l = 0.0f;  // of the lane's token; l over this lane's keys
+  as_f4 o[S::NT];                 // O^T: dims 16t + 4kg + i of token r16
+#pragma unroll
+  for (int t = 0; t < S::NT; ++t) o[t] = (as_f4){0.0f, 0.0f, 0.0f, 0.0f};
+
+  load_tile(min(wave, ntiles - 1));
+  for (int kt = wave; kt < ntiles; kt += AS_WAVES) {
+    const int p0 = kt * AC_KT;
+#pragma unroll
+    for (int j = 0; j < S::VU; ++j) {
+      const int u = lane + 64 * j, pr = u / (HD / 8), ch = u % (HD / 8);
+      *(as_u4 *)(ks + pr * S::KR + 8 * ch) = kr[j];
+      *(as_u4 *)(vs + pr * S::VR + 8 * ch) = vr[j];
+    }
+    // S^T for keys p0 + 16 t2 + 4kg + i of token r16
+    as_f4 sc[2];
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2) {
+      sc[t2] = (as_f4){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int s = 0; s < S::KS; ++s) {
+        const ac_h8 a = *(const ac_h8 *)(ks + (16 * t2 + r16) * S::KR + 32 * s + 8 * kg);
+        sc[t2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qh[s], sc[t2], 0, 0, 0);
+        sc[t2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, ql[s], sc[t2], 0, 0, 0);
+      }
+    }
+    // the next tile's loads go out now (the registers above are consumed)
+    load_tile(min(kt + AS_WAVES, ntiles - 1));
+    // A tile wholly below the block's first token's limit needs no mask.
+    if (!(p0 + AC_KT - 1 <= pos0 + t0 && p0 + AC_KT <= kend)) {  // uniform
+#pragma unroll
+      for (int t2 = 0; t2 < 2; ++t2)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int p = p0 + 16 * t2 + 4 * kg + i;
+          if (!(p <= lim && p < kend)) sc[t2][i] = -INFINITY;
+        }
+    }
+#define AC_MAX(a, b) __builtin_elementwise_maximum(a, b)
+    float mx = AC_MAX(AC_MAX(AC_MAX(sc[0][0], sc[0][1]), AC_MAX(sc[0][2], sc[0][3])),
+                      AC_MAX(AC_MAX(sc[1][0], sc[1][1]), AC_MAX(sc[1][2], sc[1][3])));
+    RowPair pr = xrow16(mx);  // the token's other keys: lanes r16 + 16 kg
+    mx = AC_MAX(pr.a, pr.b);
+    pr = xrow32(mx);
+    mx = AC_MAX(pr.a, pr.b);
+#undef AC_MAX
+    // m moves only past m + 8; mx = -inf (no key of this token in the tile)
+    // leaves it
+    const bool bump = mx > m + 8.0f;
+    const float mn = bump ? mx : m;
+    const float corr = !bump ? 1.0f : m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mn);
+    // finite, so that a token with no key yet (mn = -inf) gets 0, not NaN
+    const float mref = mn == -INFINITY ? 0.0f : mn;
+    ac_h8 ph, pl;
+    float psum = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float p = __builtin_amdgcn_exp2f(sc[j >> 2][j & 3] - mref);
+      psum += p;
+      const _Float16 h = (_Float16)p;
+      ph[j] = h;
+      if constexpr (PLO) pl[j] = (_Float16)(p - (float)h);
+    }
+    l = l * corr + psum;
+    m = mn;
+    if (!__all(corr == 1.0f)) {
+#pragma clang loop unroll(full)
+      for (int t = 0; t < S::NT; ++t)
+#pragma clang loop unroll(full)
+        for (int i = 0; i < 4; ++i) o[t][i] *= corr;
+    }
+    // V^T operand: lane s of a 16-lane group reads key rows 4kg + s/4 and
+    // 16 + 4kg + s/4, dims 16t + 4(s%4)
+    const uint16_t *va = vs + (4 * kg + (r16 >> 2)) * S::VR + 4 * (r16 & 3);
+#pragma clang loop unroll(full)
+    for (int t = 0; t < S::NT; ++t) {
+      const ac_h8 v = tr_pair((const unsigned char *)(va + 16 * t),
+                              (const unsigned char *)(va + 16 * S::VR + 16 * t));
+      o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v, ph, o[t], 0, 0, 0);
+      if constexpr (PLO) o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v, pl, o[t], 0, 0, 0);
+    }
+  }
+
+  // merge the waves: per wave (m, l, O[HD]) of its 16 tokens, in its own region
+  float *mb = (float *)vs;
+  {
+    RowPair pr = xrow16(l);
+    const float l2 = pr.a + pr.b;
+    pr = xrow32(l2);
+    if (kg == 0) {
+      mb[r16 * (HD + 2)] = m;
+      mb[r16 * (HD + 2) + 1] = pr.a + pr.b;
+    }
+#pragma unroll
+    for (int t = 0; t < S::NT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) mb[r16 * (HD + 2) + 2 + 16 * t + 4 * kg + i] = o[t][i];
+  }
+  __syncthreads();
+  const int rows = min(16, n - t0);
+  for (int idx = tid; idx < rows * HD; idx += AS_WAVES * 64) {
+    const int row = idx / HD, d = idx % HD;
+    const float *p = (const float *)ac_lds + row * (HD + 2);
+    float M = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < AS_WAVES; ++w) M = fmaxf(M, p[w * (S::WAVE / 2)]);
+    float num = 0.0f, den = 0.0f;
+#pragma unroll
+    for (int w = 0; w < AS_WAVES; ++w) {
+      const float *wb = p + w * (S::WAVE / 2);
+      const float f = wb[0] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(wb[0] - M);  // base 2
+      num = fmaf(wb[2 + d], f, num);
+      den = fmaf(wb[1], f, den);
+    }
+    out[(size_t)(t0 + row) * n_q * HD + (size_t)head * HD + d] = f2h(num / den);
+  }
+}
+
+template <int HD, bool PLO>
+static void attn_chunk_short(const void *qkv, const void *k_cache, const void *v_cache, void *out,
+                             int n_q, int n_kv, int pos0, int n, int max_seq, float scale) {
+  static bool attr = false;
+  if (!attr) {
+    (void)hipFuncSetAttribute((const void *)attn_chunk_short_kernel<HD, PLO>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, AsShape<HD>::LDS);
+    attr = true;
+  }
+  attn_chunk_short_kernel<HD, PLO>
+      <<<dim3(n_q, (n + 15) / 16), AS_WAVES * 64, AsShape<HD>::LDS, WST_STREAM>>>(
+          (const float *)qkv, (const uint16_t *)k_cache, (const uint16_t *)v_cache,
+          (uint16_t *)out, n_q, n_kv, pos0, n, max_seq, scale);
 }
 
 template <int HD, int RW, int G, bool PLO>
@@ -461,6 +702,20 @@ static void attn_chunk_mfma(const void *qkv, const void *k_cache, const void *v_
                             int plan_n) {
   const char *v = getenv("WST_ATTN_CHUNK_TG"), *pv = getenv("WST_ATTN_CHUNK_PLO");
   const bool plo = pv && pv[0] == '1';  // P as f16 hi + lo
+  // A call by itself (plan_n 0: no other launch has to give its tokens the same
+  // bits) over few positions: us, short kernel / this one, 28/4 heads of 128:
+  // 7 tokens at 100 5.5 / 6.7, at 645 9.8 / 10.1, at 1000 11.9 / 11.5; 128 at 100
+  // 7.1 / 7.7, at 300 9.1 / 9.0; 256 at 0 8.3 / 7.7. 14/2 of 64: 16 at 300 4.9 /
+  // 6.5, at 1500 9.4 / 9.6, at 2200 12.2 / 11.6; 256 at 1000 8.6 / 9.1, at 1500
+  // 10.6 / 10.5.
+  if (plan_n <= 0) {
+    if (n < 512 && (HD == 64 ? pos0 + 2 * n < 1700 : pos0 + 4 * n < 680)) {
+      (plo ? attn_chunk_short<HD, true> : attn_chunk_short<HD, false>)(
+          qkv, k_cache, v_cache, out, n_q, n_kv, pos0, n, max_seq, scale);
+      return;
+    }
+    plan_n = n;
+  }
   const int rows = n * (n_q / n_kv);
   const bool two = v && (v[0] == '1' || v[0] == '2') ? v[0] == '2'
                                                      : n_kv * ((rows + 63) / 64) >= wst_cu_count();
@@ -477,7 +732,7 @@ extern "C" wst_status_t wst_attn_chunks(const void *qkv, const void *k_cache, co
                                         void *out, int32_t n_q, int32_t n_kv, int32_t head_dim,
                                         int32_t pos0, int32_t n, int32_t max_seq, float scale,
                                         int32_t plan_n) {
-  const int pn = plan_n > 0 && plan_n < n ? plan_n : n;
+  const int pn = plan_n <= 0 ? 0 : plan_n < n ? plan_n : n;
   WST_REQUIRE(qkv && k_cache && v_cache && out, "wst_attn_chunk: null pointer");
   WST_REQUIRE(n_q > 0 && n_kv > 0 && n_q % n_kv == 0 && n > 0 && n <= 65535,
               "wst_attn_chunk: bad shape");
@@ -512,5 +767,5 @@ extern "C" wst_status_t wst_attn_chunk(const void *qkv, const void *k_cache, con
                                        void *out, int32_t n_q, int32_t n_kv, int32_t head_dim,
                                        int32_t pos0, int32_t n, int32_t max_seq, float scale) {
   return wst_attn_chunks(qkv, k_cache, v_cache, out, n_q, n_kv, head_dim, pos0, n, max_seq, scale,
-                         n);
+                         0);
 }

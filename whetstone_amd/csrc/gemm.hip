@@ -4,36 +4,35 @@
 //
 // MI355X design
 // -------------
-// * A block computes a 64-row x 64-token tile of y on MFMA
-//   (v_mfma_f32_16x16x32_f16: rows x tokens, f32 accumulate). Four waves each
-//   own 16 tokens x 64 rows (4 accumulator tiles). Measured against 128-token
-//   tiles (32 tokens per wave): fewer registers per lane and twice the blocks
-//   took the 0.5B gate|up tile from 21.3 to 18.7 us, the dequantisation being
-//   done once per 64 tokens instead of 128.
-// * K advances four int4-hier groups (128 columns) per step. The step's weights
-//   are dequantised into an f16 LDS tile exactly as the quantiser's
-//   dequantisation computes them (hier.rs:398-421: s = d*ls, m = -dmin*lm,
-//   q*s + m, each operation rounded in f32) and then rounded to f16; x is
-//   already f16. The tiles are double-buffered in LDS: the next step's packed
-//   bytes and activations are in flight while this step's 32 MFMAs per wave
-//   run, and one barrier per step separates the buffers. (With one group per
-//   step the loop was latency-bound: every step waited a full memory round
-//   trip for one group's data.)
-// * Split-K: when the output has too few tiles to fill the chip (the o and
-//   down projections of small models, any shape at few tokens), the group
-//   range is split over blocks. Each split writes its f32 partial tile to a
-//   library scratch slot, and a second kernel adds the splits in split order
-//   plus the bias and the accumulate, so the result is deterministic for a
+// * Three tile families, one choice per shape for every form (fused and
+//   unfused), so that the forms add their f32 sums alike (plan_gemm):
+//   the register tiles of gemm_tile.hpp, which dequantise into the MFMA
+//   operands, take every shape whose rows are whole 64-column halves of a
+//   128-column step; the two families here, which dequantise through LDS, take
+//   the rest: rows of other lengths, index bytes off a word, offsets past 32
+//   bits, and f16 weights with few tokens (f16_pays).
+// * gemm_mfma_kernel, 64 x 64 tiles: v_mfma_f32_16x16x32_f16 (rows x tokens,
+//   f32 accumulate), four waves of 16 tokens x 64 rows. K advances four
+//   int4-hier groups (128 columns) per step. The step's weights are dequantised
+//   into an f16 LDS tile exactly as the quantiser's dequantisation computes
+//   them (hier.rs:398-421: s = d*ls, m = -dmin*lm, q*s + m, each operation
+//   rounded in f32) and then rounded to f16; x is already f16. The tiles are
+//   double-buffered in LDS: the next step's packed bytes and activations are in
+//   flight while this step's 32 MFMAs per wave run, and one barrier per step
+//   separates the buffers. (With one group per step the loop was latency-bound:
+//   every step waited a full memory round trip for one group's data.) The fp16
+//   form (wst_gemm_fp16, the lossless reference path) copies the W tile instead.
+// * gemm_wide_kernel, 64 x 256 and 64 x 128 tiles: below.
+// * Split-K: where a grid would leave the chip idle (the o and down projections
+//   of small models, any shape at few tokens) or hold too few waves to hide its
+//   loads, the columns are split over blocks. Each split writes its f32 partial
+//   to a library scratch slot, and a second kernel adds the splits in split
+//   order plus the bias and the accumulate, so the result is deterministic for a
 //   given shape. Chunk GEMMs are never graph-captured (chunk.rs:1-12), so the
 //   slot may grow on first use.
-// * Each weight is dequantised once per 128 tokens; per step a block does
-//   8192 dequantisations against 1 M multiply-adds, so the MFMA pipe, not
-//   VALU, sets the pace.
 // * f16 rather than bf16 tiles: the same MFMA rate, three more mantissa bits
 //   (the dequantised weight rounds once, to 11 bits; products and sums are
 //   f32).
-// * The fp16 form (wst_gemm_fp16, the lossless reference path) runs the same
-//   kernel with the W tile copied instead of dequantised.
 #include "common.hpp"
 #include "gemm_tile.hpp"
 
@@ -981,11 +980,10 @@ __global__ __launch_bounds__(64 * RR_WAVES) void gemm_reduce_rope_kernel(
 }
 
 namespace {
-// The tile family: the 128 x 128 wide tiles (32x32x16 MFMA) unless
-// WST_GEMM_TILES=narrow selects the 64 x 64 tiles (16x16x32 MFMA) and
-// WST_GEMM_TILES=wide the wide tiles wherever they apply (for measurement);
-// unset, the shape picks. One choice for every chunk GEMM form, so fused and
-// unfused forms sum alike.
+// WST_GEMM_TILES (for measurement): narrow runs every chunk GEMM on the 64 x 64
+// LDS tiles, wide every int4-hier one of whole 64-column steps on the wide LDS
+// tiles; unset, the shape picks among these and the register tiles. One choice
+// for every chunk GEMM form, so fused and unfused forms sum alike.
 int gemm_tiles_mode() {  // 0 narrow, 1 by shape, 2 wide
   static int v = -1;
   if (v < 0) {
@@ -1094,13 +1092,11 @@ constexpr TileCost TILE_COST[4][4] = {  // int4, int4 SwiGLU, f16, RoPE epilogue
 // for a split a reduce launch and each further partial's way out and back (4
 // TB/s; the residual and qkv forms write one partial and reduce it anyway).
 // The partials stay below max_part bytes; the SwiGLU and RoPE epilogues never
-// split. A
-// token's bits depend on the split only, not on the tile.
+// split. A token's bits depend on the split only, not on the tile.
 // Where it lies, measured in us (big / mid / low): 896 -> 1152 x 4096 tokens
 // 20.9 / 18.7 / -; 7B gate|up x 30 53 / 40 / 26; 0.5B gate|up x 256 18 / 13.9 /
-// -, pair 12.9;
-// 896 -> 151936 x 30 49 / 28 / 22; 3584 -> 4608 x 30 unsplit low 29, split 7
-// ways 9 with its reduce.
+// -, pair 12.9; 896 -> 151936 x 30 49 / 28 / 22; 3584 -> 4608 x 30 unsplit low
+// 29, split 7 ways 9 with its reduce.
 // form: the row of TILE_COST.
 enum { FORM_INT4 = 0, FORM_SWIGLU = 1, FORM_F16 = 2, FORM_ROPE = 3 };
 void plan_tile(GemmPlan &p, int in_f, int out_f, int rows, int pn, int n, int form,
@@ -1132,21 +1128,22 @@ void plan_tile(GemmPlan &p, int in_f, int out_f, int rows, int pn, int n, int fo
   }
 }
 
-// Splits so that the grid covers the chip, each at least one step long.
-// rows: the weight matrix's row count (2 * inter for the SwiGLU form), which
-// with in_f and the plan's token count picks the tiles: the wide tiles for
-// long rows or many of them, where their deeper pipeline pays, and for any
-// shape whose 256-token tiles fill half the CUs without a split (the 0.5B
-// qkv and o projections over a 4096-token batched prefill: 30.3 -> 28.6 and
-// 25.0 -> 17.0 us, config 4 464-466k -> 475-480k tok/s); otherwise (the
-// same projections on one 256-token chunk: wide 9.0 + 3.9 us against narrow
-// 7.4 + 3.9 us for qkv) the narrow tiles, since short K split into pieces is
-// too short for the wide tiles' pipeline.
+// The family, tile and K split of a launch.
+// rows: the weight matrix's row count (2 * inter for the SwiGLU form).
+// Register tiles wherever they apply: against the LDS tiles they measured 7B
+// gate|up x 4096 1,586 -> 1,090 us, 4864 -> 896 x 256 16.9 -> 13.2, 3584 ->
+// 4608 x 5 23.8 -> 9.1, 18944 -> 3584 x 5 69 -> 17.5; slower by 3% at 2048 -> 2
+// x 5632 SwiGLU with 180 to 256 tokens.
+// Of the LDS tiles, the wide ones for long rows or many of them, where their
+// deeper pipeline pays, and for any shape whose 256-token tiles fill half the
+// CUs without a split; otherwise the narrow tiles, since short K split into
+// pieces is too short for the wide tiles' pipeline (896 -> 1152 x 256: wide
+// 9.0, narrow 7.4 us).
 // plan_n: the token count whose tiling and split-K plan the launch uses; n
 // may exceed it (several chunks in one launch): the grid then repeats the
 // plan's token tiles over n, and every token gets the bits a launch of
-// plan_n tokens gives it (the tiles are 64, 128 or 256 tokens, which divide
-// a chunk). 0: n itself.
+// plan_n tokens gives it (a token's bits depend on the K split only). 0: n
+// itself.
 GemmPlan plan_gemm(int in_f, int out_f, int n, bool hier = true, int rows = 0, bool swi = false,
                    int plan_n = 0, const void *si = nullptr,
                    size_t max_part = (size_t)256 << 20) {
@@ -1542,10 +1539,10 @@ extern "C" wst_status_t wst_gemm_hier_rope_chunk(const void *qw, const void *si,
 // wst_gemm_int4_hier_noalloc: wst_gemm_int4_hier for callers that cannot
 // allocate (graph capture, serving loops). Its split-K partials live in this
 // file-scope device array instead of the lazily allocated scratch slot. The
-// split plan splits only grids of fewer tiles than half the CUs, at most
-// ceil(CUs / tiles) ways, so the partials stay below (CUs + tiles) x (one
-// tile, at most 64 x 256 f32 = 64 KiB): under 24 MiB on 256 CUs, which this
-// array holds; a larger need is refused.
+// register tiles' plan splits no further than the array holds. The LDS tiles
+// split only grids of fewer tiles than half the CUs, at most ceil(CUs / tiles)
+// ways, so their partials stay below (CUs + tiles) x (one tile, at most 64 x 256
+// f32 = 64 KiB): under 24 MiB on 256 CUs; a larger need is refused.
 #define GM_NOALLOC_BYTES (24u << 20)
 static __device__ __align__(256) unsigned char scratch[GM_NOALLOC_BYTES];
 
