@@ -139,7 +139,10 @@ def test_gemm_rope_epilogue_equals_gemm_then_rope_cache(orc, wk, in_f, n_q, n_kv
 
 @pytest.mark.parametrize("in_f,out_f,n,accum", [(128, 1, 1, False), (192, 130, 33, True),
                                                 (896, 257, 65, False), (960, 1000, 256, True),
-                                                (4864, 96, 7, True), (256, 9000, 600, False)])
+                                                (4864, 96, 7, True), (256, 9000, 600, False),
+                                                # on the register tiles
+                                                (960, 9000, 600, True), (192, 9001, 1100, False),
+                                                (3136, 4100, 40, True)])
 def test_gemm_fp16_step_rows(orc, wk, in_f, out_f, n, accum):
     """f16 weights over the same edges: the operands are exact, so only the f32
     sums differ from float64 (at most in_f + 16 additions of relative 2^-24)."""
@@ -164,8 +167,9 @@ def test_gemm_fp16_step_rows(orc, wk, in_f, out_f, n, accum):
 
 # rows that end in half a step: each column meets its own weight once, so an
 # infinite x gives the sign's infinity and leaves the other tokens alone
-@pytest.mark.parametrize("kind", ["hier", "fp16"])
-@pytest.mark.parametrize("in_f,out_f,n", [(192, 40, 70), (960, 257, 130)])
+@pytest.mark.parametrize("kind,in_f,out_f,n", [("hier", 192, 40, 70), ("hier", 960, 257, 130),
+                                               ("fp16", 960, 9000, 600),
+                                               ("fp16", 3136, 4100, 40)])
 def test_gemm_half_step_rows_infinite_x(orc, wk, kind, in_f, out_f, n):
     print(f"{kind} gemm {in_f} -> {out_f}, {n} tokens, Inf in x", flush=True)
     rng = np.random.default_rng(66)

@@ -1099,8 +1099,8 @@ constexpr TileCost TILE_COST[4][4] = {  // int4, int4 SwiGLU, f16, RoPE epilogue
 // 29, split 7 ways 9 with its reduce.
 // form: the row of TILE_COST.
 enum { FORM_INT4 = 0, FORM_SWIGLU = 1, FORM_F16 = 2, FORM_ROPE = 3 };
-void plan_tile(GemmPlan &p, int in_f, int out_f, int rows, int pn, int n, int form,
-               size_t max_part) {
+float plan_tile(GemmPlan &p, int in_f, int out_f, int rows, int pn, int n, int form,
+                size_t max_part) {
   const bool whole = form == FORM_SWIGLU || form == FORM_ROPE;
   const int steps = (in_f + GT_KC - 1) / GT_KC, cus = wst_cu_count();
   float best = 0.0f;
@@ -1126,6 +1126,52 @@ void plan_tile(GemmPlan &p, int in_f, int out_f, int rows, int pn, int n, int fo
       }
     }
   }
+  return best;
+}
+
+// The LDS tiles' K split: a grid of fewer tiles than half the CUs, so that it
+// covers the chip, each split at least one step long.
+void split_lds(GemmPlan &p, int in_f, int out_f, int pn) {
+  const int G = in_f / HGROUP;
+  const int tiles = ((out_f + p.bm - 1) / p.bm) * ((pn + p.bn - 1) / p.bn);
+  p.splits = 1;
+  p.gps = G;
+  const int target = wst_cu_count();
+  if (tiles < target / 2) {
+    int want = (target + tiles - 1) / tiles;
+    if (gemm_split_cap() > 0) want = min(want, gemm_split_cap());
+    int g = (G + want - 1) / want;
+    g = (g + p.kg - 1) / p.kg * p.kg;
+    if ((G + g - 1) / g > GM_MAXSPLIT) g = (G + GM_MAXSPLIT - 1) / GM_MAXSPLIT;
+    g = (g + p.kg - 1) / p.kg * p.kg;
+    p.gps = g;
+    p.splits = (G + g - 1) / g;
+  }
+}
+
+// f16 weights: register tiles or the 64 x 64 LDS tiles. The register tiles' loads
+// touch 32 rows an instruction, so they pay where the LDS tiles hold several
+// blocks a CU, run long rows unsplit, or the matrix is large. Up to 64 tokens by
+// size (LDS / register tiles, us: 4864 -> 896 x 16 tokens 8.8 / 10.0, 3904 ->
+// 13620 x 4 20.1 / 22.7; but 18944 -> 3584 x 16 39 / 33, 896 -> 151936 x 16 56 /
+// 46); above, by the LDS tiles' time (0.72 us a step and block held, 3.5 fixed,
+// 3.5 for the reduce) against 1.3 times the register tiles' estimate: 1920 ->
+// 4096 x 256 14.4 / 21.5, 896 -> 4864 x 128 8.7 / 11.3; but 8192 -> 2048 x 200 44.9 /
+// 28.9, 3584 -> 4096 x 128 22.3 / 17.0, 1024 -> 16384 x 256 28.9 / 23.8, 896 ->
+// 151936 x 256 292 / 173.
+bool f16_pays(float tile_us, int in_f, int out_f, int pn) {
+  const size_t wbytes = (size_t)out_f * in_f * 2;
+  if (wbytes >= ((size_t)128 << 20)) return true;
+  if (pn <= 64) return pn > 32 && in_f >= 3072 && wbytes >= ((size_t)24 << 20);
+  GemmPlan q;
+  q.bm = GM_BM;
+  q.bn = GM_BN;
+  q.kg = GM_KG;
+  split_lds(q, in_f, out_f, pn);
+  const int blocks = ((out_f + GM_BM - 1) / GM_BM) * ((pn + GM_BN - 1) / GM_BN) * q.splits;
+  const int held = (blocks + wst_cu_count() - 1) / wst_cu_count();
+  const int steps = (q.gps + GM_KG - 1) / GM_KG;
+  return 1.3f * tile_us < 0.72f * (float)(steps * held) + (q.splits > 1 ? 7.0f : 3.5f);
 }
 
 // The family, tile and K split of a launch.
@@ -1150,16 +1196,12 @@ GemmPlan plan_gemm(int in_f, int out_f, int n, bool hier = true, int rows = 0, b
   GemmPlan p;
   if (rows <= 0) rows = out_f;
   const int pn = plan_n > 0 && plan_n < n ? plan_n : n;
-  // f16 weights for few tokens: the 64 x 64 tiles' loads, whole rows apart, are
-  // not slower there, and their K split finer (start -> tiles, us: 4864 -> 896
-  // x 16 tokens 8.8 -> 10.0, 3904 -> 13620 x 4 20.1 -> 22.7; but 18944 -> 3584
-  // x 16 39 -> 33, 896 -> 151936 x 16 56 -> 46, 4864 -> 896 x 256 19.3 -> 14.4).
-  const size_t wbytes = (size_t)rows * in_f * 2;
-  const bool f16_pays = pn > 64 || wbytes >= ((size_t)128 << 20) ||
-                        (pn > 32 && in_f >= 3072 && wbytes >= ((size_t)24 << 20));
-  if ((hier || f16_pays) && tile_ok(hier, si, in_f, out_f, rows, n)) {
-    plan_tile(p, in_f, out_f, rows, pn, n, !hier ? FORM_F16 : swi ? FORM_SWIGLU : FORM_INT4,
-              max_part);
+  float us = 0.0f;
+  const bool tiles = tile_ok(hier, si, in_f, out_f, rows, n);
+  if (tiles)
+    us = plan_tile(p, in_f, out_f, rows, pn, n, !hier ? FORM_F16 : swi ? FORM_SWIGLU : FORM_INT4,
+                   max_part);
+  if (tiles && (hier || f16_pays(us, in_f, out_f, pn))) {
     p.wide = false;
     p.nwv = 0;
     p.kg = 0;
@@ -1192,21 +1234,7 @@ GemmPlan plan_gemm(int in_f, int out_f, int n, bool hier = true, int rows = 0, b
   p.bm = p.wide ? GW_BM : GM_BM;
   p.bn = p.wide ? 32 * p.nwv : GM_BN;
   p.kg = p.wide ? GW_KG : GM_KG;
-  const int G = in_f / HGROUP;
-  const int tiles = ((out_f + p.bm - 1) / p.bm) * ((pn + p.bn - 1) / p.bn);
-  p.splits = 1;
-  p.gps = G;
-  const int target = wst_cu_count();
-  if (tiles < target / 2) {
-    int want = (target + tiles - 1) / tiles;
-    if (gemm_split_cap() > 0) want = min(want, gemm_split_cap());
-    int g = (G + want - 1) / want;
-    g = (g + p.kg - 1) / p.kg * p.kg;
-    if ((G + g - 1) / g > GM_MAXSPLIT) g = (G + GM_MAXSPLIT - 1) / GM_MAXSPLIT;
-    g = (g + p.kg - 1) / p.kg * p.kg;
-    p.gps = g;
-    p.splits = (G + g - 1) / g;
-  }
+  split_lds(p, in_f, out_f, pn);
   p.grid = dim3((out_f + p.bm - 1) / p.bm, (n + p.bn - 1) / p.bn, p.splits);
   return p;
 }
