@@ -190,9 +190,10 @@ wst_status_t wst_gemm_hier_rope_chunk(const void *qw, const void *si, const void
 /* The same four chunk GEMM forms (and the plain one) over n tokens that hold
  * several chunks, with the tiling and split-K plan of a plan_n-token chunk
  * repeated over the n tokens: each token gets the bits a call of plan_n
- * tokens gives it (n = plan_n is the call above); plan_n = 0 plans for the
- * n tokens themselves. The batched prefill uses them to run a layer's op for
- * every full chunk in one launch. */
+ * tokens gives it, whatever n (n = plan_n is the call above); plan_n = 0 plans
+ * for the n tokens themselves. The tokens go in several launches where one
+ * would pass 256 MiB of split-K partials or a kernel's 32-bit offsets. The
+ * batched prefill uses these to run a layer's op for all its chunks. */
 wst_status_t wst_gemm_int4_hier_chunks(const void *qw, const void *si, const void *sb,
                                        const void *x, const void *bias, void *y, int32_t in_f,
                                        int32_t out_f, int32_t n, int32_t accum, int32_t plan_n);
@@ -236,13 +237,13 @@ wst_status_t wst_stream_read(const void *buf, size_t bytes, void *sink);
  * forbid hipMalloc): wst_gemm_int4_hier with the same arguments and the same
  * kernels, but its split-K partial sums go to a static 24 MiB device array
  * (one per GPU, held until the process ends) instead of the library's lazily
- * allocated scratch. Nothing is allocated or freed. The sum over K is split no
- * further than the array holds (wst_gemm_int4_hier's own bound is 256 MiB, so
- * the two may add a large output in another order); a shape whose partials need
- * more all the same is refused with WST_ERR_SHAPE (none does on 256 CUs). Every call on
- * one GPU shares that array: calls that overlap on one GPU (other threads'
- * streams) race. The partials are fully written before they are read, so no
- * state carries over between calls. */
+ * allocated scratch. Nothing is allocated or freed, and the outputs are
+ * wst_gemm_int4_hier's bit for bit: the same split, with the tokens run in as many
+ * launches as the array needs. A shape of which one token's partials need more
+ * is refused with WST_ERR_SHAPE (none does on 256 CUs). Every call on one GPU
+ * shares that array: calls that overlap on one GPU (other threads' streams)
+ * race. The partials are fully written before they are read, so no state
+ * carries over between calls. */
 wst_status_t wst_gemm_int4_hier_noalloc(const void *qw, const void *si, const void *sb,
                                         const void *x, const void *bias, void *y,
                                         int32_t in_f, int32_t out_f, int32_t n, int32_t accum);

@@ -129,6 +129,79 @@ def test_gemm_rope_chunk_equals_gemm_then_rope_cache(orc, wk, in_f, n_q, n_kv, h
     assert np.array_equal(k[:, :pos0], k0[:, :pos0]) and np.array_equal(k[:, pos0 + n:], k0[:, pos0 + n:])
 
 
+def _packed(wk, in_f, out_f):
+    lin = wk.QuantLinearHier(*(wk.DeviceBuffer(k, t) for k, t in (
+        (out_f * in_f // 8, np.uint32), (out_f * in_f // 32, np.uint8), (out_f, np.uint32))),
+        in_f, out_f)
+    ffi.call("wst_fixture_pack_hier", lin.qw.ptr, lin.si.ptr, lin.sb.ptr, in_f, 0, out_f, 71, 1, 0.02)
+    return lin
+
+
+def _rows(buf, first, count, width):
+    out = np.empty(count * width, buf.dtype)
+    ffi.check(ffi.lib().wst_memcpy_d2h(out.ctypes.data, buf.at(first * width), out.nbytes))
+    return out.view(np.uint8)
+
+
+# A launch of n tokens planned for plan_n gives a token the bits of a plan_n
+# call, however large n is: past 256 MiB of K split partials (a 256-token call
+# of the first shape splits 9 ways), past 2^31 bytes of outputs (the second;
+# its SwiGLU counterpart is the third), and for the qkv form.
+@pytest.mark.parametrize("form,in_f,out_f,n,plan_n", [("norm", 18944, 3584, 2304 + 37, 256),
+                                                      ("norm", 18944, 3584, 4096, 256),
+                                                      ("plain", 18944, 3584, 2304, 256),
+                                                      ("plain", 128, 150016, 3700, 256),
+                                                      ("swiglu", 128, 75008, 7300, 256),
+                                                      ("rope", 3584, 4608, 4096 + 5, 256)])
+def test_planned_launch_gives_each_chunk_its_bits(wk, form, in_f, out_f, n, plan_n):
+    print(f"{form} {in_f} -> {out_f}, {n} tokens planned for {plan_n}", flush=True)
+    rng = np.random.default_rng(72)
+    lin = _packed(wk, in_f, 2 * out_f if form == "swiglu" else out_f)  # held: it owns the weights
+    packed = lin.qw.ptr, lin.si.ptr, lin.sb.ptr
+    x = dev_f16(wk, rng.standard_normal((n, in_f), np.float32).astype(np.float16).view(np.uint16).reshape(-1))
+    n_q, n_kv, hd = 28, 4, 128
+    if form == "norm":
+        y0 = rng.standard_normal(n * out_f, np.float32)
+        nw = dev_f16(wk, np.full(out_f, 0x3C00, np.uint16))
+        bufs = [[(wk.DeviceBuffer.from_array(y0), out_f), (wk.DeviceBuffer(n * out_f, np.float16), out_f)]
+                for _ in range(2)]
+    elif form == "rope":
+        t = np.linspace(0, 1, n * hd // 2, dtype=np.float32)
+        cos, sin = wk.DeviceBuffer.from_array(np.cos(t)), wk.DeviceBuffer.from_array(np.sin(t))
+        bufs = [[(wk.DeviceBuffer(n * out_f, np.float32), out_f)] for _ in range(2)]
+        caches = [[wk.DeviceBuffer(n_kv * n * hd, np.float16) for _ in range(2)] for _ in range(2)]
+    else:
+        t = np.float16 if form == "swiglu" else np.float32
+        bufs = [[(wk.DeviceBuffer(n * out_f, t), out_f)] for _ in range(2)]
+
+    def run(side, first, count, plan):
+        xp, o = x.at(first * in_f), [b.at(first * w) for b, w in bufs[side]]
+        if form == "norm":
+            ffi.call("wst_gemm_hier_norm_chunks", *packed, xp, None, o[0], in_f, out_f, count, 1,
+                     nw.ptr, 1e-6, o[1], plan)
+        elif form == "swiglu":
+            ffi.call("wst_gemm_hier_swiglu_chunks", *packed, xp, o[0], in_f, out_f, count, plan)
+        elif form == "rope":
+            ffi.call("wst_gemm_hier_rope_chunks", *packed, xp, None, o[0], in_f, caches[side][0].ptr,
+                     caches[side][1].ptr, cos.ptr, sin.ptr, n_q, n_kv, hd, first, count, n, None,
+                     None, 1e-6, plan)
+        else:
+            ffi.call("wst_gemm_int4_hier_chunks", *packed, xp, None, o[0], in_f, out_f, count, 0, plan)
+
+    run(0, 0, n, plan_n)
+    # the first chunk, one in the middle, and the last plan_n tokens
+    firsts = [0, n // 2 // plan_n * plan_n, n - plan_n]
+    for first in firsts:
+        run(1, first, plan_n, plan_n)
+        for (a, w), (b, _) in zip(*bufs):
+            assert np.array_equal(_rows(a, first, plan_n, w), _rows(b, first, plan_n, w)), first
+    if form == "rope":
+        for a, b in zip(*caches):
+            ca, cb = (t.numpy().view(np.uint16).reshape(n_kv, n, hd) for t in (a, b))
+            for first in firsts:
+                assert np.array_equal(ca[:, first:first + plan_n], cb[:, first:first + plan_n])
+
+
 def test_fused_chunk_forms_refuse_bad_shapes(orc, wk):
     lin = _lin(orc, wk, 51, 64, 64)
     x = _x(orc, wk, 52, 4, 64)

@@ -1,7 +1,8 @@
 """The batched prefill against the chunk-by-chunk one.
 
-A chunked prefill's full chunks go through each layer together, one launch
-per op for all of them (engine.cpp chunk_pass).
+A chunked prefill's chunks go through each layer together, one launch per op
+for all of them (engine.cpp chunk_pass); with one chunk's plan per launch (the
+first mode below) a shorter last chunk goes by itself.
 
 * WSE_CHUNK_BATCH=chunk: each launch keeps one chunk's tiling and split-K
   plan. The contract is bit-identity with running the same chunks one after
@@ -28,7 +29,7 @@ pytestmark = pytest.mark.gpu
 CFGS = {"05b_qk_rescore": dict(E.QWEN05B, qk_norm=1, rescore_k=32), "05b": E.QWEN05B,
         "7b": dict(E.QWEN7B, n_layers=4)}
 CASES = [("05b_qk_rescore", 1024), ("05b_qk_rescore", 900), ("05b", 768), ("05b", 769),
-         ("7b", 512)]
+         ("7b", 512), ("7b", 2304)]
 
 
 def _run(g, prompt, n_new, mode):

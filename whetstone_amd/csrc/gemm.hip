@@ -36,6 +36,7 @@
 #include "common.hpp"
 #include "gemm_tile.hpp"
 
+#include <algorithm>
 #include <mutex>
 
 #define HGROUP 32
@@ -1051,15 +1052,15 @@ static int gemm_bn_override() {
 }
 
 // The register tiles take rows of 128 columns or more in whole 64-column halves
-// of a step, int4-hier with 4-byte aligned index bytes, within their 32-bit
-// offsets.
-bool tile_ok(bool hier, const void *si, int in_f, int out_f, int rows, int n) {
-  const size_t lim = (size_t)1 << 31;
-  return gemm_tiles_mode() == 1 && in_f % 64 == 0 && in_f >= GT_KC &&
-         (!hier || !((uintptr_t)si & 3u)) && (size_t)n * in_f * 2 < lim &&
-         (size_t)rows * (hier ? in_f / 2 : in_f * 2) < lim &&
-         (size_t)n * out_f * 4 < lim && out_f <= (1 << 20);
+// of a step, int4-hier with 4-byte aligned index bytes, weights within their
+// 32-bit offsets. (Tokens past those go in further launches: gemm_piece.)
+bool tile_ok(bool hier, const void *si, int in_f, int rows) {
+  return gemm_tiles_mode() == 1 && in_f % 64 == 0 && in_f >= GT_KC && in_f < (1 << 29) &&
+         (!hier || !((uintptr_t)si & 3u)) &&
+         (size_t)rows * (hier ? in_f / 2 : in_f * 2) < ((size_t)1 << 31) && rows <= (1 << 20);
 }
+
+#define GM_PART_BYTES ((size_t)256 << 20)  // the scratch slot's partials
 
 // What a block of a tile costs: a step alone on its CU (lat), a step's share of
 // a CU that several blocks keep busy (thr), and launch, first loads and stores
@@ -1091,16 +1092,16 @@ constexpr TileCost TILE_COST[4][4] = {  // int4, int4 SwiGLU, f16, RoPE epilogue
 // step takes with the blocks the fullest CU holds, the tile's fixed part, and
 // for a split a reduce launch and each further partial's way out and back (4
 // TB/s; the residual and qkv forms write one partial and reduce it anyway).
-// The partials stay below max_part bytes; the SwiGLU and RoPE epilogues never
-// split. A token's bits depend on the split only, not on the tile.
+// The partials of pn tokens stay below GM_PART_BYTES; the SwiGLU and RoPE
+// epilogues never split. A token's bits depend on the split only, not on the
+// tile.
 // Where it lies, measured in us (big / mid / low): 896 -> 1152 x 4096 tokens
 // 20.9 / 18.7 / -; 7B gate|up x 30 53 / 40 / 26; 0.5B gate|up x 256 18 / 13.9 /
 // -, pair 12.9; 896 -> 151936 x 30 49 / 28 / 22; 3584 -> 4608 x 30 unsplit low
 // 29, split 7 ways 9 with its reduce.
 // form: the row of TILE_COST.
 enum { FORM_INT4 = 0, FORM_SWIGLU = 1, FORM_F16 = 2, FORM_ROPE = 3 };
-float plan_tile(GemmPlan &p, int in_f, int out_f, int rows, int pn, int n, int form,
-                size_t max_part) {
+float plan_tile(GemmPlan &p, int in_f, int out_f, int rows, int pn, int form) {
   const bool whole = form == FORM_SWIGLU || form == FORM_ROPE;
   const int steps = (in_f + GT_KC - 1) / GT_KC, cus = wst_cu_count();
   float best = 0.0f;
@@ -1110,7 +1111,7 @@ float plan_tile(GemmPlan &p, int in_f, int out_f, int rows, int pn, int n, int f
     const int tiles = ((rows + c.bm - 1) / c.bm) * ((pn + c.bn - 1) / c.bn);
     for (int want = 1; want <= (whole ? 1 : GM_MAXSPLIT) && want <= steps; ++want) {
       const int sps = (steps + want - 1) / want, splits = (steps + sps - 1) / sps;
-      if (splits > 1 && (size_t)splits * n * out_f * 4 > max_part) break;
+      if (splits > 1 && (size_t)splits * pn * out_f * 4 > GM_PART_BYTES) break;
       if (gemm_split_cap() > 0 && splits > gemm_split_cap()) break;
       const float held = (float)((tiles * splits + cus - 1) / cus);
       const float step = c.thr * held > c.lat ? c.thr * held : c.lat;
@@ -1185,37 +1186,33 @@ bool f16_pays(float tile_us, int in_f, int out_f, int pn) {
 // CUs without a split; otherwise the narrow tiles, since short K split into
 // pieces is too short for the wide tiles' pipeline (896 -> 1152 x 256: wide
 // 9.0, narrow 7.4 us).
-// plan_n: the token count whose tiling and split-K plan the launch uses; n
-// may exceed it (several chunks in one launch): the grid then repeats the
-// plan's token tiles over n, and every token gets the bits a launch of
-// plan_n tokens gives it (a token's bits depend on the K split only). 0: n
-// itself.
+// plan_n: the token count whose family, tiling and split-K plan the launch
+// uses; n may exceed it (several chunks in one launch): the grid then repeats
+// the plan's token tiles over n, and every token gets the bits a launch of
+// plan_n tokens gives it (they depend on the family and the K split only, and
+// neither on n). 0: n itself.
 GemmPlan plan_gemm(int in_f, int out_f, int n, bool hier = true, int rows = 0, bool swi = false,
-                   int plan_n = 0, const void *si = nullptr,
-                   size_t max_part = (size_t)256 << 20) {
+                   int plan_n = 0, const void *si = nullptr) {
   GemmPlan p;
   if (rows <= 0) rows = out_f;
   const int pn = plan_n > 0 && plan_n < n ? plan_n : n;
   float us = 0.0f;
-  const bool tiles = tile_ok(hier, si, in_f, out_f, rows, n);
+  const bool tiles = tile_ok(hier, si, in_f, rows);
   if (tiles)
-    us = plan_tile(p, in_f, out_f, rows, pn, n, !hier ? FORM_F16 : swi ? FORM_SWIGLU : FORM_INT4,
-                   max_part);
+    us = plan_tile(p, in_f, out_f, rows, pn, !hier ? FORM_F16 : swi ? FORM_SWIGLU : FORM_INT4);
   if (tiles && (hier || f16_pays(us, in_f, out_f, pn))) {
     p.wide = false;
     p.nwv = 0;
     p.kg = 0;
-    p.grid = dim3((unsigned)(((rows + p.bm - 1) / p.bm) * ((n + p.bn - 1) / p.bn)), p.splits, 1);
     return p;
   }
   p.tile = TILE_OLD;
-  // (The wide tiles address x with 32-bit byte offsets, and step through it
-  // 64 columns at a time: in_f must be whole steps.)
+  // (The wide tiles step through x 64 columns at a time: in_f must be whole
+  // steps.)
   const int tm = gemm_tiles_mode();
   const int rows_t256 = ((rows + GW_BM - 1) / GW_BM) * ((pn + 255) / 256);
-  p.wide = hier && tm > 0 && in_f % GW_KC == 0 &&
-           (tm == 2 || in_f >= 2048 || rows >= 4096 || rows_t256 >= wst_cu_count() / 2) &&
-           (size_t)n * in_f * 2 < ((size_t)1 << 31);
+  p.wide = hier && tm > 0 && in_f % GW_KC == 0 && in_f < (1 << 29) &&
+           (tm == 2 || in_f >= 2048 || rows >= 4096 || rows_t256 >= wst_cu_count() / 2);
   // Wide tiles of 128 tokens for the split-K shapes (256-token tiles fewer
   // than half the CUs), where 256-token tiles would leave CUs without a
   // tile: 7B qkv 43.0 -> 36.2 us, 7B down 100.3 -> 95.6 us (0.5B down
@@ -1235,8 +1232,28 @@ GemmPlan plan_gemm(int in_f, int out_f, int n, bool hier = true, int rows = 0, b
   p.bn = p.wide ? 32 * p.nwv : GM_BN;
   p.kg = p.wide ? GW_KG : GM_KG;
   split_lds(p, in_f, out_f, pn);
-  p.grid = dim3((out_f + p.bm - 1) / p.bm, (n + p.bn - 1) / p.bn, p.splits);
   return p;
+}
+
+// The grid of a launch over n tokens. rows as in plan_gemm.
+void set_grid(GemmPlan &p, int rows, int n) {
+  const int mb = (rows + p.bm - 1) / p.bm, nb = (n + p.bn - 1) / p.bn;
+  p.grid = p.tile != TILE_OLD ? dim3((unsigned)(mb * nb), p.splits, 1) : dim3(mb, nb, p.splits);
+}
+
+// How many of n tokens one launch takes: within the register and wide tiles'
+// 32-bit offsets and with its partials (parts a token: the K splits, or one for
+// a form that reduces from the scratch in any case; 0: none) in part_bytes,
+// though at least one. In whole token tiles where it is less than n.
+int gemm_piece(const GemmPlan &p, int in_f, int out_f, int n, int parts,
+               size_t part_bytes = GM_PART_BYTES) {
+  const size_t lim = ((size_t)1 << 31) - 1;
+  size_t most = (size_t)n;
+  if (p.tile != TILE_OLD || p.wide) most = std::min(most, lim / ((size_t)in_f * 2));
+  if (p.tile != TILE_OLD) most = std::min(most, lim / ((size_t)out_f * 4));
+  if (parts > 0) most = std::min(most, part_bytes / ((size_t)parts * out_f * 4));
+  if (most < (size_t)n && most >= (size_t)p.bn) most -= most % p.bn;
+  return most > 0 ? (int)most : 1;
 }
 
 template <class S, int EPI, bool TAIL, bool F16>
@@ -1318,18 +1335,15 @@ void launch_gemm(const GemmPlan &p, const void *w, const void *si, const void *s
         (const uint16_t *)bias, (float *)y, ws, in_f, out_f, n, accum, p.gps);
 }
 
-// The GEMM into the split scratch (always, even with one split): the fused
-// reduce kernels read it.
-wst_status_t gemm_to_scratch(const void *w, const void *si, const void *sb, const void *x,
-                             int in_f, int out_f, int n, float **ws_out, int *splits_out,
-                             int plan_n = 0) {
-  const GemmPlan p = plan_gemm(in_f, out_f, n, true, 0, false, plan_n, si);
+// The GEMM of n tokens (one piece) into the split scratch (always, even with
+// one split): the fused reduce kernels read it.
+float *gemm_to_scratch(GemmPlan &p, const void *w, const void *si, const void *sb, const void *x,
+                       int in_f, int out_f, int n) {
   float *ws = (float *)wst_static_scratch(WST_SCRATCH_GEMM, (size_t)p.splits * n * out_f * 4);
-  if (!ws) return WST_ERR_OOM;
+  if (!ws) return nullptr;
+  set_grid(p, out_f, n);
   launch_gemm<true, false>(p, w, si, sb, x, nullptr, nullptr, ws, in_f, out_f, n, 0);
-  *ws_out = ws;
-  *splits_out = p.splits;
-  return WST_OK;
+  return ws;
 }
 }  // namespace
 
@@ -1339,33 +1353,35 @@ wst_status_t wst_gemm_mfma(bool hier, const void *w, const void *si, const void 
                            const void *x, const void *bias, void *y, int32_t in_f, int32_t out_f,
                            int32_t n, int32_t accum, float *ws_ext, size_t ws_cap,
                            int32_t plan_n) {
-  const GemmPlan p = plan_gemm(in_f, out_f, n, hier, 0, false, plan_n, si,
-                               ws_ext ? ws_cap : (size_t)256 << 20);
-  const int splits = p.splits;
+  GemmPlan p = plan_gemm(in_f, out_f, n, hier, 0, false, plan_n, si);
+  const int splits = p.splits, parts = splits > 1 ? splits : 0;
+  const int piece = gemm_piece(p, in_f, out_f, n, parts, ws_ext ? ws_cap : GM_PART_BYTES);
   float *ws = nullptr;
   if (splits > 1) {
-    const size_t need = (size_t)splits * n * out_f * 4;
-    if (ws_ext) {
-      if (need > ws_cap) {
-        snprintf(wst_err_buf, sizeof(wst_err_buf),
-                 "split-K partials need %zu bytes, above the %zu-byte static scratch", need, ws_cap);
-        return WST_ERR_SHAPE;
-      }
-      ws = ws_ext;
-    } else {
-      ws = (float *)wst_static_scratch(WST_SCRATCH_GEMM, need);
-      if (!ws) return WST_ERR_OOM;
+    const size_t need = (size_t)parts * piece * out_f * 4;
+    if (ws_ext && need > ws_cap) {
+      snprintf(wst_err_buf, sizeof(wst_err_buf),
+               "split-K partials need %zu bytes, above the %zu-byte static scratch", need, ws_cap);
+      return WST_ERR_SHAPE;
     }
+    ws = ws_ext ? ws_ext : (float *)wst_static_scratch(WST_SCRATCH_GEMM, need);
+    if (!ws) return WST_ERR_OOM;
   }
-  if (hier)
-    launch_gemm<true, false>(p, w, si, sb, x, bias, y, ws, in_f, out_f, n, accum);
-  else
-    launch_gemm<false, false>(p, w, nullptr, nullptr, x, bias, y, ws, in_f, out_f, n, accum);
-  if (splits > 1) {
-    const size_t total = (size_t)n * out_f;
-    const int blocks = (int)((total + 255) / 256 < 4096 ? (total + 255) / 256 : 4096);
-    gemm_split_reduce_kernel<<<blocks, 256, 0, WST_STREAM>>>(ws, (const uint16_t *)bias,
-                                                              (float *)y, out_f, n, splits, accum);
+  for (int s = 0; s < n; s += piece) {
+    const int k = min(piece, n - s);
+    const void *xs = (const uint16_t *)x + (size_t)s * in_f;
+    float *ys = (float *)y + (size_t)s * out_f;
+    set_grid(p, out_f, k);
+    if (hier)
+      launch_gemm<true, false>(p, w, si, sb, xs, bias, ys, ws, in_f, out_f, k, accum);
+    else
+      launch_gemm<false, false>(p, w, nullptr, nullptr, xs, bias, ys, ws, in_f, out_f, k, accum);
+    if (splits > 1) {
+      const size_t total = (size_t)k * out_f;
+      const int blocks = (int)((total + 255) / 256 < 4096 ? (total + 255) / 256 : 4096);
+      gemm_split_reduce_kernel<<<blocks, 256, 0, WST_STREAM>>>(ws, (const uint16_t *)bias, ys,
+                                                                out_f, k, splits, accum);
+    }
   }
   return WST_OK;
 }
@@ -1396,14 +1412,17 @@ extern "C" wst_status_t wst_gemm_hier_swiglu_chunks(const void *qw, const void *
   WST_REQUIRE(act, "wst_gemm_hier_swiglu_chunk: null pointer");
   // Never split: a tile pairs BM/2 gate rows with the matching up rows.
   GemmPlan p = plan_gemm(in_f, inter, n, true, 2 * inter, true, plan_n, si);
-  if (p.tile != TILE_OLD) {
-    p.grid = dim3((unsigned)(((inter + p.bm / 2 - 1) / (p.bm / 2)) * ((n + p.bn - 1) / p.bn)), 1, 1);
-  } else {
+  if (p.tile == TILE_OLD) {
     p.splits = 1;
     p.gps = in_f / HGROUP;
-    p.grid = dim3((inter + p.bm / 2 - 1) / (p.bm / 2), (n + p.bn - 1) / p.bn, 1);
   }
-  launch_gemm<true, true>(p, qw, si, sb, x, nullptr, act, nullptr, in_f, inter, n, 0);
+  const int piece = gemm_piece(p, in_f, inter, n, 0);
+  for (int s = 0; s < n; s += piece) {
+    const int k = min(piece, n - s);
+    set_grid(p, 2 * inter, k);
+    launch_gemm<true, true>(p, qw, si, sb, (const uint16_t *)x + (size_t)s * in_f, nullptr,
+                            (uint16_t *)act + (size_t)s * inter, nullptr, in_f, inter, k, 0);
+  }
   WST_TRY_KERNEL("wst_gemm_hier_swiglu_chunk");
   return WST_OK;
 }
@@ -1423,32 +1442,37 @@ extern "C" wst_status_t wst_gemm_hier_norm_chunks(const void *qw, const void *si
   if (st != WST_OK) return st;
   WST_REQUIRE(y && norm_w && h_out, "wst_gemm_hier_norm_chunk: null pointer");
   WST_REQUIRE(out_f <= 16384, "wst_gemm_hier_norm_chunk: out_features above 16384");
-  float *ws;
-  int splits;
-  st = gemm_to_scratch(qw, si, sb, x, in_f, out_f, n, &ws, &splits, plan_n);
-  if (st != WST_OK) return st;
   static bool attr = false;
   if (!attr) {
     (void)hipFuncSetAttribute((const void *)gemm_reduce_norm_kernel<0>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, 16384 * 4);
     attr = true;
   }
-  if (out_f % 8 == 0 && out_f <= 4096 && !(((uintptr_t)y | (uintptr_t)h_out | (uintptr_t)norm_w |
-                                              (uintptr_t)bias) & 15u)) {
-    const int threads = 64 * ((out_f / 8 + 63) / 64);
-    gemm_reduce_norm8_kernel<<<n, threads, 0, WST_STREAM>>>(
-        ws, (const uint16_t *)bias, (float *)y, out_f, n, splits, accum, (const uint16_t *)norm_w,
-        eps, (uint16_t *)h_out);
-    WST_TRY_KERNEL("wst_gemm_hier_norm_chunk");
-    return WST_OK;
+  GemmPlan p = plan_gemm(in_f, out_f, n, true, 0, false, plan_n, si);
+  const int piece = gemm_piece(p, in_f, out_f, n, p.splits);
+  for (int s = 0; s < n; s += piece) {
+    const int k = min(piece, n - s);
+    float *ys = (float *)y + (size_t)s * out_f;
+    uint16_t *hs = (uint16_t *)h_out + (size_t)s * out_f;
+    float *ws =
+        gemm_to_scratch(p, qw, si, sb, (const uint16_t *)x + (size_t)s * in_f, in_f, out_f, k);
+    if (!ws) return WST_ERR_OOM;
+    if (out_f % 8 == 0 && out_f <= 4096 && !(((uintptr_t)y | (uintptr_t)h_out | (uintptr_t)norm_w |
+                                                (uintptr_t)bias) & 15u)) {
+      const int threads = 64 * ((out_f / 8 + 63) / 64);
+      gemm_reduce_norm8_kernel<<<k, threads, 0, WST_STREAM>>>(ws, (const uint16_t *)bias, ys, out_f,
+                                                              k, p.splits, accum,
+                                                              (const uint16_t *)norm_w, eps, hs);
+      continue;
+    }
+    auto kern = out_f <= 1024   ? gemm_reduce_norm_kernel<2>
+                : out_f <= 2048 ? gemm_reduce_norm_kernel<4>
+                : out_f <= 4096 ? gemm_reduce_norm_kernel<8>
+                                : gemm_reduce_norm_kernel<0>;
+    kern<<<k, 512, (size_t)out_f * 4, WST_STREAM>>>(ws, (const uint16_t *)bias, ys, out_f, k,
+                                                    p.splits, accum, (const uint16_t *)norm_w, eps,
+                                                    hs);
   }
-  auto kern = out_f <= 1024   ? gemm_reduce_norm_kernel<2>
-              : out_f <= 2048 ? gemm_reduce_norm_kernel<4>
-              : out_f <= 4096 ? gemm_reduce_norm_kernel<8>
-                              : gemm_reduce_norm_kernel<0>;
-  kern<<<n, 512, (size_t)out_f * 4, WST_STREAM>>>(ws, (const uint16_t *)bias, (float *)y, out_f, n,
-                                                  splits, accum, (const uint16_t *)norm_w, eps,
-                                                  (uint16_t *)h_out);
   WST_TRY_KERNEL("wst_gemm_hier_norm_chunk");
   return WST_OK;
 }
@@ -1498,53 +1522,55 @@ extern "C" wst_status_t wst_gemm_hier_rope_chunks(const void *qw, const void *si
   // + 21.1 us in two launches, 7B over 1000 tokens 58 + 18). Unsplit tiles all
   // give the same bits, so their choice here is free. The QK-norm of a
   // 128-wide head would sum over two waves: those take the reduce kernel.
-  {
-    GemmPlan p = plan_gemm(in_f, out_f, n, true, 0, false, plan_n, si);
-    if (p.tile != TILE_OLD && p.splits == 1 && rope_epilogue_on() &&
-        (head_dim == 64 || (head_dim == 128 && !q_norm_w && !k_norm_w)) &&
-        (size_t)max_seq * head_dim * 2 < ((size_t)1 << 31)) {
-      plan_tile(p, in_f, out_f, out_f, n, n, FORM_ROPE, 0);
-      p.grid = dim3((unsigned)(((out_f + p.bm - 1) / p.bm) * ((n + p.bn - 1) / p.bn)), 1, 1);
+  GemmPlan p = plan_gemm(in_f, out_f, n, true, 0, false, plan_n, si);
+  const bool epilogue = p.tile != TILE_OLD && p.splits == 1 && rope_epilogue_on() &&
+                        (head_dim == 64 || (head_dim == 128 && !q_norm_w && !k_norm_w)) &&
+                        (size_t)max_seq * head_dim * 2 < ((size_t)1 << 31);
+  if (epilogue) plan_tile(p, in_f, out_f, out_f, n, FORM_ROPE);
+  const int piece = gemm_piece(p, in_f, out_f, n, epilogue ? 0 : p.splits);
+  for (int s = 0; s < n; s += piece) {
+    const int k = min(piece, n - s), at = pos0 + s;
+    const void *xs = (const uint16_t *)x + (size_t)s * in_f;
+    float *ys = (float *)qkv + (size_t)s * out_f;
+    if (epilogue) {
+      set_grid(p, out_f, k);
       const GtRope re{(uint16_t *)k_cache, (uint16_t *)v_cache, (const float *)cos_tab,
                       (const float *)sin_tab, (const uint16_t *)q_norm_w,
-                      (const uint16_t *)k_norm_w, n_q, n_kv, pos0, max_seq, eps};
+                      (const uint16_t *)k_norm_w, n_q, n_kv, at, max_seq, eps};
       auto go = [&](auto shape) {
         if (head_dim == 64)
-          launch_tile<decltype(shape), GT_ROPE64>(p, qw, si, sb, x, bias, qkv, nullptr, in_f,
-                                                  out_f, out_f, n, 0, re);
+          launch_tile<decltype(shape), GT_ROPE64>(p, qw, si, sb, xs, bias, ys, nullptr, in_f, out_f,
+                                                  out_f, k, 0, re);
         else
-          launch_tile<decltype(shape), GT_ROPE128>(p, qw, si, sb, x, bias, qkv, nullptr, in_f,
-                                                   out_f, out_f, n, 0, re);
+          launch_tile<decltype(shape), GT_ROPE128>(p, qw, si, sb, xs, bias, ys, nullptr, in_f,
+                                                   out_f, out_f, k, 0, re);
       };
       if (p.tile == TILE_BIG) go(GtBig{});
       else if (p.tile == TILE_MID) go(GtMidPair{});
       else go(GtLowPair{});
-      WST_TRY_KERNEL("wst_gemm_hier_rope_chunk");
-      return WST_OK;
+      continue;
     }
-  }
-  float *ws;
-  int splits;
-  st = gemm_to_scratch(qw, si, sb, x, in_f, out_f, n, &ws, &splits, plan_n);
-  if (st != WST_OK) return st;
+    const float *ws = gemm_to_scratch(p, qw, si, sb, xs, in_f, out_f, k);
+    if (!ws) return WST_ERR_OOM;
 #define RR_LAUNCH(NARROW_, G_)                                                                 \
   do {                                                                                       \
-    const int items_ = n * ((n_q + n_kv + (G_) - 1) / (G_));                                 \
+    const int items_ = k * ((n_q + n_kv + (G_) - 1) / (G_));                                 \
     gemm_reduce_rope_kernel<NARROW_, G_><<<(items_ + RR_WAVES - 1) / RR_WAVES, 64 * RR_WAVES, 0, \
                                            WST_STREAM>>>(                                    \
-        ws, (const uint16_t *)bias, (float *)qkv, splits, n, (uint16_t *)k_cache,            \
+        ws, (const uint16_t *)bias, ys, p.splits, k, (uint16_t *)k_cache,                    \
         (uint16_t *)v_cache, (const float *)cos_tab, (const float *)sin_tab, n_q, n_kv,       \
-        head_dim, pos0, max_seq, (const uint16_t *)q_norm_w, (const uint16_t *)k_norm_w, eps); \
+        head_dim, at, max_seq, (const uint16_t *)q_norm_w, (const uint16_t *)k_norm_w, eps);  \
   } while (0)
-  const bool big = n >= 1024;
-  if (head_dim <= 64) {
-    if (big) RR_LAUNCH(true, 8);
-    else RR_LAUNCH(true, 1);
-  } else {
-    if (big) RR_LAUNCH(false, 8);
-    else RR_LAUNCH(false, 1);
-  }
+    const bool big = k >= 1024;
+    if (head_dim <= 64) {
+      if (big) RR_LAUNCH(true, 8);
+      else RR_LAUNCH(true, 1);
+    } else {
+      if (big) RR_LAUNCH(false, 8);
+      else RR_LAUNCH(false, 1);
+    }
 #undef RR_LAUNCH
+  }
   WST_TRY_KERNEL("wst_gemm_hier_rope_chunk");
   return WST_OK;
 }
@@ -1566,11 +1592,11 @@ extern "C" wst_status_t wst_gemm_hier_rope_chunk(const void *qw, const void *si,
 //
 // wst_gemm_int4_hier_noalloc: wst_gemm_int4_hier for callers that cannot
 // allocate (graph capture, serving loops). Its split-K partials live in this
-// file-scope device array instead of the lazily allocated scratch slot. The
-// register tiles' plan splits no further than the array holds. The LDS tiles
-// split only grids of fewer tiles than half the CUs, at most ceil(CUs / tiles)
-// ways, so their partials stay below (CUs + tiles) x (one tile, at most 64 x 256
-// f32 = 64 KiB): under 24 MiB on 256 CUs; a larger need is refused.
+// file-scope device array instead of the lazily allocated scratch slot, as many
+// tokens a launch as the array holds (gemm_piece): the plan, and so the sum, is
+// the other entry's. (One token's partials: at most 16 splits of fewer than
+// 2^20 outputs, and a grid that wide is not split that far; a larger need is
+// refused.)
 #define GM_NOALLOC_BYTES (24u << 20)
 static __device__ __align__(256) unsigned char scratch[GM_NOALLOC_BYTES];
 

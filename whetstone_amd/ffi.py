@@ -151,6 +151,11 @@ ABI = {
     "wst_gemm_hier_norm_chunk": (I32, [P, P, P, P, P, P, I32, I32, I32, I32, P, F32, P]),
     "wst_gemm_hier_rope_chunk": (I32, [P, P, P, P, P, P, I32, P, P, P, P, I32, I32, I32, I32, I32,
                                        I32, P, P, F32]),
+    "wst_gemm_int4_hier_chunks": (I32, [P, P, P, P, P, P, I32, I32, I32, I32, I32]),
+    "wst_gemm_hier_swiglu_chunks": (I32, [P, P, P, P, P, I32, I32, I32, I32]),
+    "wst_gemm_hier_norm_chunks": (I32, [P, P, P, P, P, P, I32, I32, I32, I32, P, F32, P, I32]),
+    "wst_gemm_hier_rope_chunks": (I32, [P, P, P, P, P, P, I32, P, P, P, P, I32, I32, I32, I32, I32,
+                                        I32, P, P, F32, I32]),
 }
 
 
