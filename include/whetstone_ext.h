@@ -235,7 +235,7 @@ wst_status_t wst_stream_read(const void *buf, size_t bytes, void *sink);
 /* No counterpart in the reference. For callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): wst_gemm_int4_hier with the same arguments and the same
- * kernels, but its split-K partial sums go to a static 24 MiB device array
+ * kernels, but its split-K partial sums go to a static 64 MiB device array
  * (one per GPU, held until the process ends) instead of the library's lazily
  * allocated scratch. Nothing is allocated or freed, and the outputs are
  * wst_gemm_int4_hier's bit for bit: the same split, with the tokens run in as many

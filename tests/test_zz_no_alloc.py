@@ -1,11 +1,11 @@
 """wst_gemm_int4_hier_noalloc (the split-K chunk GEMM with its partials in a
 static device array) against wst_gemm_int4_hier, through the C ABI.
 
-Two calls in a row on the same GPU, the second with a smaller input, each
+Calls in a row on the same GPU, the second with a smaller input, each
 compared bit for bit with the allocating entry point on the same inputs (the
 same kernels and the same split plan, so the same f32 sums in the same
-order), and with a float64 product of the dequantised weights. Both shapes
-split K (too few output tiles to fill the chip), so the static array is used.
+order), and with a float64 product of the dequantised weights. Every shape
+splits K (too few output tiles to fill the chip), so the static array is used.
 """
 import numpy as np
 import pytest
@@ -41,11 +41,19 @@ def _case(orc, wk, in_f, out_f, n, seed, accum):
 
 
 def test_noalloc_gemm_equals_allocating_gemm_twice(orc, wk):
-    # the 0.5B down projection over a 256-token chunk: long rows, so the
-    # 64 x 256 tiles, 14 of them, K split 16 ways (14.7 MB of partials)
+    # the 0.5B down projection over a 256-token chunk: register tiles of 128
+    # rows x 64 tokens, K split 8 ways (7.3 MB of partials)
     _case(orc, wk, 4864, 896, 256, 11, accum=True)
-    # then a smaller input on the same static array: 64 x 64 tiles, K split
+    # then a smaller input on the same static array
     _case(orc, wk, 896, 200, 37, 12, accum=False)
+
+
+@pytest.mark.parametrize("in_f,out_f,n,accum", [
+    (4096, 2176, 4000, True),  # 2 splits, 66.4 MiB of partials: two launches
+    (2080, 200, 37, True)])    # rows of an odd number of groups: the 64 x 64 LDS tiles
+def test_noalloc_gemm_equals_allocating_gemm(orc, wk, in_f, out_f, n, accum):
+    print(f"no-allocation gemm {in_f} -> {out_f}, {n} tokens", flush=True)
+    _case(orc, wk, in_f, out_f, n, 13, accum)
 
 
 def test_noalloc_gemm_argument_checks(wk):

@@ -1594,10 +1594,13 @@ extern "C" wst_status_t wst_gemm_hier_rope_chunk(const void *qw, const void *si,
 // allocate (graph capture, serving loops). Its split-K partials live in this
 // file-scope device array instead of the lazily allocated scratch slot, as many
 // tokens a launch as the array holds (gemm_piece): the plan, and so the sum, is
-// the other entry's. (One token's partials: at most 16 splits of fewer than
+// the other entry's. 64 MiB hold those of any layer of the two configured
+// models at up to 1,024 tokens (18944 -> 3584: 31.5 at 256, 61 at 896), so only
+// larger calls pay for a second launch: at 24 MiB 256 tokens took 91 us and 1000
+// took 285, in one launch 56 and 159. (One token's partials: at most 16 splits of fewer than
 // 2^20 outputs, and a grid that wide is not split that far; a larger need is
 // refused.)
-#define GM_NOALLOC_BYTES (24u << 20)
+#define GM_NOALLOC_BYTES (64u << 20)
 static __device__ __align__(256) unsigned char scratch[GM_NOALLOC_BYTES];
 
 // The array's device address, looked up once per device with that device
