@@ -216,7 +216,8 @@ wst_status_t wst_gemm_hier_rope_chunks(const void *qw, const void *si, const voi
 /* wst_attn_chunk over n tokens that hold several chunks, each token with the
  * bits a call of plan_n tokens gives it whatever its position (the planned count
  * picks how the keys are split into partial sums). plan_n = 0 is wst_attn_chunk:
- * a call by itself, which also takes another kernel over few positions. */
+ * a call by itself, which also takes another kernel over few positions (where no
+ * other call has to give the same bits). */
 wst_status_t wst_attn_chunks(const void *qkv, const void *k_cache, const void *v_cache,
                              void *out, int32_t n_q, int32_t n_kv, int32_t head_dim,
                              int32_t pos0, int32_t n, int32_t max_seq, float scale,

@@ -23,6 +23,7 @@ import pytest
 
 from conftest import ns_tol
 from whetstone_amd import engine as E
+from whetstone_amd import ffi
 
 pytestmark = pytest.mark.gpu
 
@@ -105,3 +106,62 @@ def test_batched_prefill_planned_whole_matches_chunk_by_chunk(cfg_name, n_prompt
         dk = float(np.max(np.abs(a[3][k].astype(np.float64) - b[3][k])))
         print(f"  step {k}: logits {dk:.3g} apart, top-2 margin {_top2(a[3][k]):.3g}")
         assert _top2(a[3][k]) < 2 * ns_tol(a[3][k]), (k, _top2(a[3][k]))
+
+
+def _chunk_by_calls(wk, g, cfg, caches, ids, pos0, max_seq):
+    """A chunk pass as the ABI's calls, each by itself: the rows' logits."""
+    H, hd, nq, nkv, I, V = (cfg[k] for k in ("hidden", "head_dim", "n_q", "n_kv", "inter", "vocab"))
+    n, nqkv, eps = len(ids), (nq + 2 * nkv) * hd, cfg["eps"]
+    vec = {}
+
+    def v(name):
+        if name not in vec:
+            vec[name] = wk.DeviceBuffer.from_array(g.vector_host(name).view(np.float16))
+        return vec[name].ptr
+
+    def w(name):
+        return g.tensor(name)[:3]
+
+    rope = wk.RopeTable(max_seq, hd, cfg["rope_theta"])
+    tok = wk.DeviceBuffer.from_array(np.asarray(ids, np.int32))
+    x, qkv, logits = (wk.DeviceBuffer(n * k, np.float32) for k in (H, nqkv, V))
+    h, attn, act = (wk.DeviceBuffer(n * k, np.float16) for k in (H, nq * hd, I))
+    ffi.call("wst_embed_int4_hier_chunk", *w("embed"), tok.ptr, x.ptr, H, V, n)
+    ffi.call("wst_rmsnorm_chunk", x.ptr, v("L0.in_norm"), h.ptr, H, n, eps)
+    for l in range(cfg["n_layers"]):
+        k, c = caches[l]
+        nxt = "final_norm" if l + 1 == cfg["n_layers"] else f"L{l + 1}.in_norm"
+        ffi.call("wst_gemm_hier_rope_chunk", *w(f"L{l}.qkv"), h.ptr, v(f"L{l}.qkv_bias"), qkv.ptr, H,
+                 k.ptr, c.ptr, rope.cos.ptr, rope.sin.ptr, nq, nkv, hd, pos0, n, max_seq, None,
+                 None, eps)
+        ffi.call("wst_attn_chunk", qkv.ptr, k.ptr, c.ptr, attn.ptr, nq, nkv, hd, pos0, n, max_seq,
+                 1.0 / np.sqrt(hd))
+        ffi.call("wst_gemm_hier_norm_chunk", *w(f"L{l}.o"), attn.ptr, None, x.ptr, nq * hd, H, n, 1,
+                 v(f"L{l}.post_norm"), eps, h.ptr)
+        ffi.call("wst_gemm_hier_swiglu_chunk", *w(f"L{l}.gate_up"), h.ptr, act.ptr, H, I, n)
+        ffi.call("wst_gemm_hier_norm_chunk", *w(f"L{l}.down"), act.ptr, None, x.ptr, I, H, n, 1,
+                 v(nxt), eps, h.ptr)
+    ffi.call("wst_gemm_int4_hier", *w("embed"), h.ptr, None, logits.ptr, H, V, n, 0)
+    return logits.numpy().reshape(n, V)
+
+
+# An engine's chunk is the ABI's calls, each by itself, so it runs whichever
+# kernel is the faster one for that chunk (a short cache's attention too): a
+# prompt, then a few tokens behind it, short and long caches on both sides of
+# the attention's rule at head_dim 128 (680 positions).
+@pytest.mark.parametrize("hd,first,chunk", [(64, 16, 5), (64, 100, 5), (128, 16, 5), (128, 250, 7)])
+def test_a_chunk_equals_the_calls_one_by_one(wk, hd, first, chunk):
+    cfg = dict(n_layers=2, hidden=512, n_q=512 // hd, n_kv=2, head_dim=hd, inter=1024, vocab=8192,
+               tied=1, qkv_bias=1, qk_norm=0, rescore_k=0, eps=1e-6, rope_theta=1e6)
+    print(f"chunks of {first} and {chunk} tokens, head_dim {hd}", flush=True)
+    max_seq = first + chunk + 3
+    g = E.Model(cfg, seed=5)
+    eng = E.Engine(g, max_seq)
+    ids = np.random.default_rng(6).integers(0, cfg["vocab"], first + chunk).astype(np.int32)
+    caches = [[wk.DeviceBuffer(2 * max_seq * hd, np.float16) for _ in range(2)] for _ in range(2)]
+    for part, pos0 in ((ids[:first], 0), (ids[first:], first)):
+        eng.forward_chunk(part)
+        want = _chunk_by_calls(wk, g, cfg, caches, part, pos0, max_seq)
+        assert np.array_equal(eng.logits().view(np.uint32), want[-1].view(np.uint32)), pos0
+    eng.close()
+    g.close()

@@ -910,11 +910,13 @@ struct ChunkBufs {
 // plan_n is the token count the GEMMs' tiling and split-K plan is made for:
 // n (plan_n = 0) lets a launch over many chunks drop the split-K that one
 // chunk's few tiles need; plan_n = width keeps one chunk's plan, so that every
-// token gets the bits the chunk-by-chunk pass gives it. A chunk's attention
-// reads the cache only up to its own last position, so the later chunks' K/V
-// rows already in the cache are never read.
+// token gets the bits the chunk-by-chunk pass gives it. attn_plan is the
+// attention's: 0 where no other pass has to give the same bits, so that a short
+// cache takes the kernel that is the faster one there (wst_attn_chunks). A
+// chunk's attention reads the cache only up to its own last position, so the
+// later chunks' K/V rows already in the cache are never read.
 static wst_status_t chunk_pass(wse_engine *e, const int32_t *ids, int n, bool want_logits,
-                               int width, int plan_n, const ChunkBufs &b) {
+                               int width, int plan_n, int attn_plan, const ChunkBufs &b) {
   const wse_model &m = *e->m;
   const wse_config_t &c = m.c;
   const int H = c.hidden, hd = c.head_dim, nq = c.n_q, nkv = c.n_kv, I = c.inter, V = c.vocab;
@@ -954,7 +956,7 @@ static wst_status_t chunk_pass(wse_engine *e, const int32_t *ids, int n, bool wa
                                eps));
     }
     TRY(wst_attn_chunks(b.qkv, e->kc[(size_t)l], e->vc[(size_t)l], b.attn, nq, nkv, hd, pos0, n,
-                        e->max_seq, scale, pn));
+                        e->max_seq, scale, attn_plan));
     TRY(wst_gemm_hier_norm_chunks(L.o.qw, L.o.si, L.o.sb, b.attn, nullptr, b.x, nq * hd, H, n, 1,
                                   L.post_norm, eps, b.h, pn));
     TRY(wst_gemm_hier_swiglu_chunks(L.gate_up.qw, L.gate_up.si, L.gate_up.sb, b.h, b.act, H, I,
@@ -988,11 +990,6 @@ static wst_status_t chunk_pass(wse_engine *e, const int32_t *ids, int n, bool wa
   return wse_engine_set_pos(e, pos0 + n);
 }
 
-static wst_status_t forward_chunk(wse_engine *e, const int32_t *ids, int n, bool want_logits) {
-  const ChunkBufs b{e->c_tokens, e->c_x, e->c_h, e->c_qkv, e->c_attn, e->c_act};
-  return chunk_pass(e, ids, n, want_logits, e->chunk_width, 0, b);
-}
-
 // The batched prefill's buffers, grown to n tokens.
 static wst_status_t ensure_batch(wse_engine *e, int n) {
   if (e->b_cap >= n) return WST_OK;
@@ -1015,13 +1012,20 @@ static wst_status_t ensure_batch(wse_engine *e, int n) {
 // with n > width), planned for the whole launch (1, the default: a shorter last
 // chunk goes along, 7B prefill of 1000 tokens 20.9 -> 17.0 ms);
 // WSE_CHUNK_BATCH=chunk keeps one chunk's plan per launch (bit-identical to
-// the chunk-by-chunk pass); WSE_CHUNK_BATCH=0 runs the chunks one by one.
+// the chunk-by-chunk pass); WSE_CHUNK_BATCH=0 runs the chunks one by one. Those
+// two plan the attention by the chunk; the default leaves it to the launch.
 enum BatchMode { BATCH_OFF, BATCH_WHOLE, BATCH_CHUNK_PLAN };
 static BatchMode chunk_batch_mode() {
   const char *v = getenv("WSE_CHUNK_BATCH");
   if (!v || !v[0]) return BATCH_WHOLE;
   if (v[0] == '0') return BATCH_OFF;
   return strcmp(v, "chunk") == 0 ? BATCH_CHUNK_PLAN : BATCH_WHOLE;
+}
+
+static wst_status_t forward_chunk(wse_engine *e, const int32_t *ids, int n, bool want_logits) {
+  const ChunkBufs b{e->c_tokens, e->c_x, e->c_h, e->c_qkv, e->c_attn, e->c_act};
+  return chunk_pass(e, ids, n, want_logits, e->chunk_width, 0,
+                    chunk_batch_mode() == BATCH_WHOLE ? 0 : n, b);
 }
 
 wst_status_t wse_engine_max_seq(const wse_engine_t *e, int32_t *out) {
@@ -1092,7 +1096,8 @@ wst_status_t wse_engine_prefill(wse_engine_t *e, const int32_t *ids, int32_t n, 
     if (mode != BATCH_OFF && (batch >= 2 * w || (mode == BATCH_WHOLE && n > w))) {
       TRY(ensure_batch(e, (batch + w - 1) / w * w));
       const ChunkBufs b{e->b_tokens, e->b_x, e->b_h, e->b_qkv, e->b_attn, e->b_act};
-      TRY(chunk_pass(e, ids, batch, batch == n, w, mode == BATCH_CHUNK_PLAN ? w : 0, b));
+      const int plan = mode == BATCH_CHUNK_PLAN ? w : 0;
+      TRY(chunk_pass(e, ids, batch, batch == n, w, plan, plan, b));
       s = batch;
     }
     for (; s < n; s += w) {
