@@ -198,6 +198,25 @@ def test_gemm_half_step_rows_infinite_x(orc, wk, kind, in_f, out_f, n):
     assert np.all(np.isfinite(np.delete(got, tok, axis=0)))
 
 
+# a row whose scale is infinite stays infinite: the columns past its end add no
+# 0 * Inf (rows of half a step, of a whole number of steps, of odd group counts)
+@pytest.mark.parametrize("in_f,n", [(192, 5), (960, 70), (896, 70), (1248, 70)])
+def test_gemm_infinite_scale_stays_infinite(wk, in_f, n):
+    print(f"gemm {in_f} columns, an infinite scale, {n} tokens", flush=True)
+    out_f, bad = 130, 129
+    qw = wk.DeviceBuffer.from_array(np.full(out_f * in_f // 8, 0x77777777, np.uint32))
+    si = wk.DeviceBuffer.from_array(np.full(out_f * in_f // 32, 0x11, np.uint8))
+    d = np.full(out_f, 0x2000, np.uint32)  # d 2^-7, dmin 0
+    d[bad] = 0x7C00
+    sb = wk.DeviceBuffer.from_array(d)
+    x = dev_f16(wk, np.full(n * in_f, 0x3C00, np.uint16))
+    y = wk.DeviceBuffer(n * out_f, np.float32)
+    ffi.call("wst_gemm_int4_hier", qw.ptr, si.ptr, sb.ptr, x.ptr, None, y.ptr, in_f, out_f, n, 0)
+    got = y.numpy().reshape(n, out_f)
+    assert np.all(got[:, bad] == np.inf)
+    assert np.all(np.delete(got, bad, axis=1) == 7 * in_f / 128)  # (exact in f32)
+
+
 @pytest.mark.parametrize("hd,n_q,n_kv,pos0,n", [(64, 14, 2, 1702, 37), (128, 28, 4, 900, 37),
                                                 (128, 28, 4, 5, 37)])
 def test_attn_chunk_output_between_words(orc, wk, hd, n_q, n_kv, pos0, n):

@@ -233,8 +233,8 @@ __global__ __launch_bounds__(S::THREADS, S::MT * S::NT > 8 ? 1 : 2) void gemm_ti
   // The step's eight MFMA k-steps i (groups 2 (i / 4) + half, word i % 4):
   // the next k-step's operands are read and dequantised under this one's
   // MFMAs.
-  // A tail step's index bytes sit in the upper half of the word, and its groups
-  // 2 and 3 read scales of zero above it.
+  // A tail step's index bytes sit in the upper half of the word; its groups 2
+  // and 3 are weights of zero, also in a row whose d or dmin is not finite.
   auto compute = [&](const GtW<MT, F16> &w, int buf, int st) {
     const int sh = 8 * half + (TAIL && st == whole ? 16 : 0);
     const unsigned char *xb = gt_lds + buf * S::XBUF + xbase;
@@ -248,6 +248,7 @@ __global__ __launch_bounds__(S::THREADS, S::MT * S::NT > 8 ? 1 : 2) void gemm_ti
         sc[f] = ds[f] * (float)(ix & 0xFu);
         sc16[f] = sc[f] * 0.0625f;
         mm[f] = dm[f] * (float)((ix >> 4) & 0xFu);
+        if (TAIL && s == 1 && st == whole) sc[f] = sc16[f] = mm[f] = 0.0f;
       }
     };
     auto read_x = [&](int i) {
