@@ -74,6 +74,45 @@ def test_gemm_step_rows(orc, wk, in_f, out_f, n, accum):
     assert np.array_equal(got[n], y0.reshape(n + 1, out_f)[n])  # nothing past the last token
 
 
+def _off_a_word(wk, lin):
+    """The index bytes at an odd address: the register tiles refuse them."""
+    si = lin.si.numpy()
+    return wk.DeviceBuffer.from_array(np.concatenate([np.zeros(1, np.uint8), si]))
+
+
+# the wide LDS tiles, which take what the register tiles refuse: index bytes off
+# a word (off 1) and rows of one 64-column step (off 0). 256-token tiles split and
+# not, 128-token tiles split and not, the last tile ragged in both directions,
+# fewer steps than the kernel's four in flight
+@pytest.mark.parametrize("in_f,out_f,n,accum,off", [(2112, 130, 37, True, 1), (1536, 8260, 100, False, 1),
+                                                    (2048, 300, 300, False, 1), (2048, 2100, 520, True, 1),
+                                                    (128, 4100, 300, False, 1), (64, 4100, 70, True, 0)])
+def test_gemm_wide_tiles(orc, wk, in_f, out_f, n, accum, off):
+    print(f"wide tiles {in_f} -> {out_f}, {n} tokens", flush=True)
+    lin, w, x, xd, bias, bd = _operands(orc, wk, in_f, out_f, n, 69)
+    si = _off_a_word(wk, lin)
+    y0 = orc.fixture_normal(69, 4, (n + 1) * out_f, 1.0)
+    y = wk.DeviceBuffer.from_array(y0.copy())
+    ffi.call("wst_gemm_int4_hier", lin.qw.ptr, si.at(1) if off else lin.si.ptr, lin.sb.ptr, xd.ptr,
+             bd.ptr, y.ptr, in_f, out_f, n, int(accum))
+    got = y.numpy().astype(np.float64).reshape(n + 1, out_f)
+    y0 = y0.reshape(n + 1, out_f)
+    ref = x @ w.T + bias + (y0[:n] if accum else 0.0)
+    _check(got[:n], x, w, ref)
+    assert np.array_equal(got[n], y0[n])  # nothing past the last token
+
+
+@pytest.mark.parametrize("in_f,inter,n,off", [(2048, 70, 300, 1), (896, 4099, 40, 1), (64, 2050, 257, 0)])
+def test_gemm_swiglu_wide_tiles(orc, wk, in_f, inter, n, off):
+    print(f"wide gate|up {in_f} -> {inter}, {n} tokens", flush=True)
+    lin, w, x, xd, _, _ = _operands(orc, wk, in_f, 2 * inter, n, 70)
+    si = _off_a_word(wk, lin)
+    act = wk.DeviceBuffer.from_array(np.full((n + 1) * inter, 7.0, np.float16))
+    ffi.call("wst_gemm_hier_swiglu_chunk", lin.qw.ptr, si.at(1) if off else lin.si.ptr, lin.sb.ptr,
+             xd.ptr, act.ptr, in_f, inter, n)
+    _check_swiglu(act.numpy().astype(np.float64).reshape(n + 1, inter), x, w, inter, n)
+
+
 @pytest.mark.parametrize("in_f,inter,n", [(128, 1, 1), (256, 128, 128), (896, 161, 129),
                                           (384, 700, 300), (192, 100, 40), (320, 4000, 300)])
 def test_gemm_swiglu_step_rows(orc, wk, in_f, inter, n):
@@ -82,7 +121,10 @@ def test_gemm_swiglu_step_rows(orc, wk, in_f, inter, n):
     act = wk.DeviceBuffer.from_array(np.full((n + 1) * inter, 7.0, np.float16))
     ffi.call("wst_gemm_hier_swiglu_chunk", lin.qw.ptr, lin.si.ptr, lin.sb.ptr, xd.ptr, act.ptr,
              in_f, inter, n)
-    got = act.numpy().astype(np.float64).reshape(n + 1, inter)
+    _check_swiglu(act.numpy().astype(np.float64).reshape(n + 1, inter), x, w, inter, n)
+
+
+def _check_swiglu(got, x, w, inter, n):
     gu = x @ w.T
     err = 2.0 * 2.0 ** -11 * (np.abs(x) @ np.abs(w).T) + 1e-5
     g, u = gu[:, :inter], gu[:, inter:]

@@ -9,8 +9,8 @@
 //   the register tiles of gemm_tile.hpp, which dequantise into the MFMA
 //   operands, take every shape whose rows are whole 64-column halves of a
 //   128-column step; the two families here, which dequantise through LDS, take
-//   the rest: rows of other lengths, index bytes off a word, offsets past 32
-//   bits, and f16 weights with few tokens (f16_pays).
+//   the rest: rows of other lengths, index bytes off a word, weights past 32-bit
+//   offsets or 2^20 rows, and f16 weights with few tokens (f16_pays).
 // * gemm_mfma_kernel, 64 x 64 tiles: v_mfma_f32_16x16x32_f16 (rows x tokens,
 //   f32 accumulate), four waves of 16 tokens x 64 rows. K advances four
 //   int4-hier groups (128 columns) per step. The step's weights are dequantised
@@ -345,8 +345,10 @@ __global__ __launch_bounds__(GM_THREADS) void gemm_mfma_kernel(
 //   sixteen destination registers in every round). A 128-row variant (four
 //   accumulator tiles a wave, 168 VGPRs) broke this: one ring register was
 //   renamed across the loop's back edge and rows 96..127 of some tiles came
-//   out wrong (tests/test_gpu_kernels.py's 896 -> 33000 case caught it). It
-//   is not built.
+//   out wrong. It is not built. tests/test_build_isa.py reads the registers off
+//   the compiler's output, and tests/test_gpu_gemm_shapes.py runs the tiles on
+//   what still reaches them (plan_gemm): index bytes off a word, rows of one
+//   64-column step.
 // * K advances two groups (64 columns) per step; split-K and the epilogue
 //   (through LDS, token-major) are those of gemm_mfma_kernel. SWI: rows
 //   0..31 of a tile are gate rows a0..a0+31 and rows 32..63 the up rows
