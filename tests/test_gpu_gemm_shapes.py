@@ -277,14 +277,16 @@ def test_attn_chunk_output_between_words(orc, wk, hd, n_q, n_kv, pos0, n):
     assert np.array_equal(*res)
 
 
+@pytest.mark.parametrize("planned", [False, True])
 @pytest.mark.parametrize("hd,n_q,n_kv,pos0,n", [(128, 28, 4, 645, 7), (128, 28, 4, 652, 7),
                                                 (128, 8, 8, 1001, 256), (128, 4, 2, 0, 131),
                                                 (128, 4, 4, 0, 1), (64, 14, 2, 300, 33),
                                                 (64, 8, 8, 1687, 6), (64, 8, 8, 1688, 6),
                                                 (64, 14, 2, 677, 511), (64, 14, 2, 0, 512)])
-def test_attn_chunk_positions(orc, wk, hd, n_q, n_kv, pos0, n):
-    """Both kernels on both sides of the rule that picks one, a wave's last tiles
-    empty or partly attended, NaN past the attended end, against float64.
+def test_attn_chunk_positions(orc, wk, hd, n_q, n_kv, pos0, n, planned):
+    """Both kernels on both sides of the rule that picks one (planned calls stay
+    on the shared-tile kernel), a wave's last tiles empty or partly attended,
+    NaN past the attended end, against float64.
 
     Bound: P is rounded to f16 (2^-11 of each weight), the scores keep 22 bits
     of |q||k| (scores of order 1: 2^-13 allowed), the output is rounded to f16."""
@@ -298,8 +300,8 @@ def test_attn_chunk_positions(orc, wk, hd, n_q, n_kv, pos0, n):
     kd, vd = (dev_f16(wk, t.view(np.uint16).reshape(-1)) for t in (k, v))
     qd = wk.DeviceBuffer.from_array(qkv.reshape(-1))
     out = wk.DeviceBuffer(n * n_q * hd, np.float16)
-    ffi.call("wst_attn_chunk", qd.ptr, kd.ptr, vd.ptr, out.ptr, n_q, n_kv, hd, pos0, n, max_seq,
-             hd ** -0.5)
+    ffi.call("wst_attn_chunks", qd.ptr, kd.ptr, vd.ptr, out.ptr, n_q, n_kv, hd, pos0, n, max_seq,
+             hd ** -0.5, n if planned else 0)
     got = out.numpy().astype(np.float64).reshape(n, n_q, hd)
     for h in range(n_q):
         kh, vh = (t[h // g, :pos0 + n].astype(np.float64) for t in (k, v))

@@ -527,8 +527,8 @@ def test_gemm_fp16_matches_matmul(orc, wk, in_f, out_f, n):
 
 
 def _with_tg(tg, fn):
-    """Runs fn with the chunk attention's token groups per wave forced (1 or
-    2; None: the library's choice by token count)."""
+    """Runs fn with the chunk attention's row waves per key group forced (1 or
+    2; None: the library's choice by the row count)."""
     if tg is None:
         return fn()
     os.environ["WST_ATTN_CHUNK_TG"] = str(tg)
@@ -538,7 +538,18 @@ def _with_tg(tg, fn):
         os.environ.pop("WST_ATTN_CHUNK_TG", None)
 
 
-@pytest.mark.parametrize("tg", [1, 2])
+def _chunk_attention(tg, qd, cache, out, n_q, n_kv, hd, pos0, n, max_seq, scale):
+    """tg None: wst_attn_chunk, a call by itself (over few positions the short
+    kernel). 1 or 2: wst_attn_chunks planned for its own tokens, which stays on
+    the shared-tile kernel, with 32 or 64 (token, head) rows a block."""
+    args = (qd.ptr, cache.k.ptr, cache.v.ptr, out.ptr, n_q, n_kv, hd, pos0, n, max_seq, scale)
+    if tg is None:
+        ffi.call("wst_attn_chunk", *args)
+    else:
+        _with_tg(tg, lambda: ffi.call("wst_attn_chunks", *args, n))
+
+
+@pytest.mark.parametrize("tg", [None, 1, 2])
 @pytest.mark.parametrize("n_q,n_kv,hd,pos0,n,max_seq", [
     (14, 2, 64, 0, 256, 256), (14, 2, 64, 1000, 44, 1100), (28, 4, 128, 0, 256, 300),
     (28, 4, 128, 3840, 256, 4096), (8, 8, 128, 5, 1, 16), (7, 1, 64, 2000, 37, 2100)])
@@ -546,7 +557,7 @@ def test_chunk_attention_equals_per_token_decode_attention(orc, wk, n_q, n_kv, h
                                                            max_seq, tg):
     """Chunk attention (chunk_ops.cu:187-265) is decode attention per token:
     token j attends to cache positions [0, pos0 + j] (chunk_kernels.rs:262-360).
-    Both token groupings of the MFMA kernel (16 or 32 tokens per block)."""
+    Both MFMA kernels, and both row groupings of the shared-tile one."""
     rng = np.random.default_rng(pos0 + n + hd)
     kc = f16(orc, rng.standard_normal(n_kv * max_seq * hd).astype(np.float32))
     vc = f16(orc, rng.standard_normal(n_kv * max_seq * hd).astype(np.float32))
@@ -558,8 +569,7 @@ def test_chunk_attention_equals_per_token_decode_attention(orc, wk, n_q, n_kv, h
     qd = wk.DeviceBuffer.from_array(qkv)
     out = wk.DeviceBuffer(n * n_q * hd, np.float16)
     scale = np.float32(1.0 / math.sqrt(hd))
-    _with_tg(tg, lambda: ffi.call("wst_attn_chunk", qd.ptr, cache.k.ptr, cache.v.ptr, out.ptr,
-                                  n_q, n_kv, hd, pos0, n, max_seq, scale))
+    _chunk_attention(tg, qd, cache, out, n_q, n_kv, hd, pos0, n, max_seq, scale)
     got = out.numpy().astype(np.float64).reshape(n, n_q * hd)
     for j in range(n):
         want = np.empty(n_q * hd, np.uint16)
@@ -568,7 +578,7 @@ def test_chunk_attention_equals_per_token_decode_attention(orc, wk, n_q, n_kv, h
         assert np.max(np.abs(got[j] - orc.f16_value(want))) < 2e-3, j
 
 
-@pytest.mark.parametrize("tg", [1, 2])
+@pytest.mark.parametrize("tg", [None, 1, 2])
 @pytest.mark.parametrize("n_q,n_kv,hd,pos0,n,max_seq", [
     (14, 2, 64, 0, 256, 300), (28, 4, 128, 1000, 44, 1100), (14, 2, 64, 45, 256, 301),
     (28, 4, 128, 7, 20, 61)])
@@ -597,8 +607,7 @@ def test_chunk_attention_ignores_nonfinite_past_the_attended_end(orc, wk, n_q, n
     scale = np.float32(1.0 / math.sqrt(hd))
     print(f"chunk attention with NaN/Inf past position {kend}: n_q {n_q} hd {hd} pos0 {pos0} "
           f"n {n} max_seq {max_seq} tg {tg}", flush=True)
-    _with_tg(tg, lambda: ffi.call("wst_attn_chunk", qd.ptr, cache.k.ptr, cache.v.ptr, out.ptr,
-                                  n_q, n_kv, hd, pos0, n, max_seq, scale))
+    _chunk_attention(tg, qd, cache, out, n_q, n_kv, hd, pos0, n, max_seq, scale)
     got = out.numpy().astype(np.float64).reshape(n, n_q * hd)
     assert np.all(np.isfinite(got))
     for j in range(n):
@@ -610,14 +619,16 @@ def test_chunk_attention_ignores_nonfinite_past_the_attended_end(orc, wk, n_q, n
 
 
 @pytest.mark.parametrize("n_q,n_kv,hd,pos0,n", [(14, 2, 64, 0, 1536), (28, 4, 128, 300, 700),
-                                               (7, 1, 64, 33, 517)])
+                                               (7, 1, 64, 33, 517), (14, 2, 64, 300, 256),
+                                               (8, 8, 64, 1000, 200), (28, 4, 128, 0, 40)])
 def test_chunk_attention_token_groupings_are_bit_identical(orc, wk, n_q, n_kv, hd, pos0, n):
-    """A token's output does not depend on how many tokens share its block
-    (16 or 32): its valid keys are in the same tiles, taken by the same wave in
-    the same order, and a block's extra tiles are wholly masked for it. So the
-    library may pick the grouping by token count (a batched prefill and the
-    same chunks one by one get the same bits). Long prompts (the default picks
-    32 here) also checked against decode attention on a sample of tokens."""
+    """A token's output does not depend on how many rows share its block (32 or
+    64 (token, head) rows): its valid keys are in the same tiles, taken by the
+    same key group in the same order, and a block's extra tiles are wholly
+    masked for it. So the library may pick the grouping by the row count (a
+    batched prefill and the same chunks one by one get the same bits). With four
+    key groups and, at head_dim 64 for up to 256 tokens past position 128, with
+    eight. Also checked against decode attention on a sample of tokens."""
     max_seq = pos0 + n + 9
     rng = np.random.default_rng(n + hd)
     kc = f16(orc, rng.standard_normal(n_kv * max_seq * hd).astype(np.float32))
@@ -633,8 +644,8 @@ def test_chunk_attention_token_groupings_are_bit_identical(orc, wk, n_q, n_kv, h
     for tg in (1, 2, None):
         out = wk.DeviceBuffer(n * n_q * hd, np.float16)
         print(f"chunk attention tg {tg}: n_q {n_q} hd {hd} pos0 {pos0} n {n}", flush=True)
-        _with_tg(tg, lambda: ffi.call("wst_attn_chunk", qd.ptr, cache.k.ptr, cache.v.ptr,
-                                      out.ptr, n_q, n_kv, hd, pos0, n, max_seq, scale))
+        _with_tg(tg, lambda: ffi.call("wst_attn_chunks", qd.ptr, cache.k.ptr, cache.v.ptr,
+                                      out.ptr, n_q, n_kv, hd, pos0, n, max_seq, scale, n))
         outs[tg] = out.numpy().view(np.uint16).copy()
     assert np.array_equal(outs[1], outs[2]), int(np.sum(outs[1] != outs[2]))
     assert np.array_equal(outs[None], outs[2])
@@ -644,3 +655,31 @@ def test_chunk_attention_token_groupings_are_bit_identical(orc, wk, n_q, n_kv, h
         q = np.ascontiguousarray(qkv[j * row:j * row + n_q * hd])
         orc.lib().orc_attn_decode(q, kc, vc, want, n_q, n_kv, hd, pos0 + j, max_seq, scale)
         assert np.max(np.abs(got[j] - orc.f16_value(want))) < 2e-3, j
+
+
+@pytest.mark.parametrize("n_q,n_kv,hd,pos0,n,plan_n", [(14, 2, 64, 0, 700, 256), (14, 2, 64, 77, 130, 32),
+                                                       (8, 8, 64, 1500, 600, 200),
+                                                       (28, 4, 128, 0, 600, 256),
+                                                       (28, 4, 128, 500, 100, 7)])
+def test_planned_chunk_attention_equals_its_chunks(orc, wk, n_q, n_kv, hd, pos0, n, plan_n):
+    """n tokens planned for plan_n get the bits that calls of plan_n tokens (the
+    last one shorter, planned alike) give them, at every position."""
+    max_seq, row = pos0 + n + 9, (n_q + 2 * n_kv) * hd
+    rng = np.random.default_rng(n + plan_n)
+    kc, vc = (f16(orc, rng.standard_normal(n_kv * max_seq * hd).astype(np.float32)) for _ in range(2))
+    cache = wk.KvCache(n_kv, n_q, hd, max_seq)
+    cache.k.copy_from(kc.view(np.float16))
+    cache.v.copy_from(vc.view(np.float16))
+    qd = wk.DeviceBuffer.from_array((rng.standard_normal(n * row) * 2).astype(np.float32))
+    whole, parts = (wk.DeviceBuffer(n * n_q * hd, np.float16) for _ in range(2))
+    print(f"planned chunk attention: n_q {n_q} hd {hd} pos0 {pos0} n {n} plan {plan_n}", flush=True)
+
+    def call(out, first, count):
+        ffi.call("wst_attn_chunks", qd.at(first * row), cache.k.ptr, cache.v.ptr,
+                 out.at(first * n_q * hd), n_q, n_kv, hd, pos0 + first, count, max_seq,
+                 1.0 / math.sqrt(hd), plan_n)
+
+    call(whole, 0, n)
+    for first in range(0, n, plan_n):
+        call(parts, first, min(plan_n, n - first))
+    assert np.array_equal(whole.numpy().view(np.uint16), parts.numpy().view(np.uint16))
