@@ -33,8 +33,8 @@ def test_gemm_swiglu_chunk_equals_gemm_then_swiglu(orc, wk, in_f, inter, n, exac
     one K order). The fused form never splits K; where the unfused one does
     (few output tiles: the fourth case), its f32 sums are added in another
     order, and the f16 outputs may differ in the last place. The last case
-    runs 512 tokens in one call, as a batched prefill does: 260 x 2 tiles of
-    128 rows, so both forms take the 128-row wide tiles."""
+    runs 512 tokens in one call, as a batched prefill does. The two forms may
+    take tiles of different sizes; a token's sum does not depend on them."""
     lin = _lin(orc, wk, 21, in_f, 2 * inter)
     x = _x(orc, wk, 22, n, in_f)
     gu = wk.DeviceBuffer(n * 2 * inter, np.float32)
@@ -91,12 +91,11 @@ def test_gemm_norm_chunk_equals_gemm_then_rmsnorm(orc, wk, in_f, out_f, n, accum
 def test_gemm_rope_chunk_equals_gemm_then_rope_cache(orc, wk, in_f, n_q, n_kv, hd, pos0, n, qk,
                                                      has_bias):
     """The fused qkv form against the GEMM then wst_rope_cache_chunk, bit for
-    bit (q rotated, k and v as computed, the cache rows). At head_dim 64 with
-    about 1800 tokens or more the GEMM runs unsplit on 256-token tiles, one
-    head a tile, and the tile's epilogue does the norm, rotation and append
-    (the last three cases: one with a ragged last tile, one without a bias,
-    as Qwen3's projections have none, ending at the cache's last row); below
-    that a reduce kernel does them after the GEMM."""
+    bit (q rotated, k and v as computed, the cache rows). Where the GEMM runs
+    unsplit, the tile's epilogue does the norm (at head_dim 64), rotation and
+    append (the last three cases: one with a ragged last tile, one without a
+    bias, as Qwen3's projections have none, ending at the cache's last row);
+    where its K is split a reduce kernel does them after the GEMM."""
     out_f = (n_q + 2 * n_kv) * hd
     max_seq = pos0 + n + (7 if has_bias else 0)
     lin = _lin(orc, wk, 41, in_f, out_f)
