@@ -171,11 +171,11 @@ __global__ __launch_bounds__(256) void attn_chunk_kernel(
 // accumulator, exponentials, P.V: about 0.5 us for a wave alone) where a CU
 // holds few waves, and MFMA and VALU issue (12 32-clk MFMAs and ~100 VALU ops a
 // tile at head_dim 64) where it is full: 128 VGPRs at head_dim 64 keep four
-// waves a SIMD (135 kept three: 77 against 65 us). Measured in us against 16 or
-// 32 tokens of one head a block with K and V staged through registers (heads,
-// head_dim, tokens at position): 14/2 of 64, 4096 at 0: 79 -> 63; 14/2 of 64,
-// 256 at 3840: 21.8 -> 18.3; 28/4 of 128, 243 at 1792: 33 -> 21; 28/4 of 128,
-// 4096 at 0: 285 -> 245, 1000 at 0: 39 -> 33. Over few positions the
+// waves a SIMD (135 kept three: 77 against 65 us). Measured in us, calls in a row,
+// against 16 or 32 tokens of one head a block with K and V staged through
+// registers (heads, head_dim, tokens at position): 14/2 of 64, 4096 at 0: 71 ->
+// 58; 14/2 of 64, 256 at 3840: 19.8 -> 16.9; 28/4 of 128, 243 at 1792: 29.0 ->
+// 18.5; 28/4 of 128, 4096 at 0: 256 -> 215, 1000 at 0: 31.5 -> 26.9. Over few positions the
 // launch's fixed parts count and the short kernel below is the faster one.
 typedef _Float16 ac_h8 __attribute__((ext_vector_type(8)));
 typedef short ac_s4 __attribute__((ext_vector_type(4)));
@@ -704,9 +704,9 @@ static void attn_chunk_mfma(const void *qkv, const void *k_cache, const void *v_
   const bool plo = pv && pv[0] == '1';  // P as f16 hi + lo
   // A call by itself (plan_n 0: no other launch has to give its tokens the same
   // bits) over few positions: us, short kernel / this one, 28/4 heads of 128:
-  // 7 tokens at 100 5.5 / 6.7, at 645 9.8 / 10.1, at 1000 11.9 / 11.5; 128 at 100
-  // 7.1 / 7.7, at 300 9.1 / 9.0; 256 at 0 8.3 / 7.7. 14/2 of 64: 16 at 300 4.9 /
-  // 6.5, at 1500 9.4 / 9.6, at 2200 12.2 / 11.6; 256 at 1000 8.6 / 9.1, at 1500
+  // 7 tokens at 100 5.5 / 6.8, at 645 8.5 / 10.1, at 1000 11.9 / 11.5; 128 at 100
+  // 7.0 / 7.8, at 300 9.1 / 9.0; 256 at 0 8.3 / 7.7. 14/2 of 64: 16 at 300 5.4 /
+  // 6.7, at 1500 9.4 / 9.7, at 2200 12.2 / 11.6; 256 at 1000 8.9 / 9.3, at 1500
   // 10.6 / 10.5.
   if (plan_n <= 0) {
     if (n < 512 && (HD == 64 ? pos0 + 2 * n < 1700 : pos0 + 4 * n < 680)) {
