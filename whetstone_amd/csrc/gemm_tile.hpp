@@ -105,7 +105,7 @@ struct GtW {
 // tiles vary fastest. 32-bit offsets: n in_f 2, rows in_f / 2 and n out_f 4
 // are below 2^31 (the host checks).
 // TAIL: rows end in half a step (in_f % 128 == 64): the last step has groups 0
-// and 1 only; its groups 2 and 3 are weights of zero.
+// and 1 only and skips the other four of its eight k-steps.
 // F16: w is f16 [rows][in_f] (si and sb unused): a lane's operand is 16 bytes of
 // a row, loaded straight into registers; k-step i covers columns 16 i .. 16 i +
 // 15.
@@ -233,8 +233,9 @@ __global__ __launch_bounds__(S::THREADS, S::MT * S::NT > 8 ? 1 : 2) void gemm_ti
   // The step's eight MFMA k-steps i (groups 2 (i / 4) + half, word i % 4):
   // the next k-step's operands are read and dequantised under this one's
   // MFMAs.
-  // A tail step's index bytes sit in the upper half of the word; its groups 2
-  // and 3 are weights of zero, also in a row whose d or dmin is not finite.
+  // A tail step's index bytes sit in the upper half of the word, and its last
+  // four k-steps are left out: nothing past a row's end is multiplied (zeros in
+  // their place would make NaN of an infinite x or scale).
   auto compute = [&](const GtW<MT, F16> &w, int buf, int st) {
     const int sh = 8 * half + (TAIL && st == whole ? 16 : 0);
     const unsigned char *xb = gt_lds + buf * S::XBUF + xbase;
@@ -248,29 +249,22 @@ __global__ __launch_bounds__(S::THREADS, S::MT * S::NT > 8 ? 1 : 2) void gemm_ti
         sc[f] = ds[f] * (float)(ix & 0xFu);
         sc16[f] = sc[f] * 0.0625f;
         mm[f] = dm[f] * (float)((ix >> 4) & 0xFu);
-        if (TAIL && s == 1 && st == whole) sc[f] = sc16[f] = mm[f] = 0.0f;
       }
     };
     auto read_x = [&](int i) {
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
-        gt_u4 v = *(const gt_u4 *)(xb + t * 32 * GT_XROW +
-                                   (xsw ^ (uint32_t)((F16 ? 2 * i : 8 * (i >> 2) + (i & 3)) * 16)));
-        // (a tail step's second half: x of zero too, as 0 * Inf is NaN)
-        if (TAIL && i >= 4) v &= (gt_u4)(st == whole ? 0u : ~0u);
-        xf[i & 1][t] = __builtin_bit_cast(gt_h8, v);
+        xf[i & 1][t] = *(const gt_h8 *)(xb + t * 32 * GT_XROW +
+                                        (xsw ^ (uint32_t)((F16 ? 2 * i : 8 * (i >> 2) + (i & 3)) * 16)));
       }
     };
     auto make_w = [&](int i) {
 #pragma unroll
       for (int f = 0; f < MT; ++f) {
-        if constexpr (F16) {
-          // (a tail step's second half: weights of zero)
-          const uint32_t keep = TAIL && st == whole && i >= 4 ? 0u : ~0u;
-          wf[i & 1][f] = __builtin_bit_cast(gt_h8, TAIL ? w.q[f][i] & (gt_u4)keep : w.q[f][i]);
-        } else {
+        if constexpr (F16)
+          wf[i & 1][f] = __builtin_bit_cast(gt_h8, w.q[f][i]);
+        else
           wf[i & 1][f] = gt_dequant(w.q[f][i >> 2][i & 3], sc[f], sc16[f], mm[f]);
-        }
       }
     };
     scales(0);
@@ -282,6 +276,7 @@ __global__ __launch_bounds__(S::THREADS, S::MT * S::NT > 8 ? 1 : 2) void gemm_ti
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
+      if (TAIL && i == 4 && st == whole) break;  // (uniform)
       if (i < 7) {
         read_x(i + 1);
         if (i == 3) scales(1);
